@@ -250,7 +250,7 @@ __global__ void __launch_bounds__(64 * WAVES, 8 / WAVES)
   }
 }
 // ---------------------------------------------------------------- per chain
-// One wave per chain, element e in lane e % 64, slot e / 64 (4 slots).
+// One block of 256 threads per chain, thread e holds state element e.
 __device__ inline void split_bf16(float v, __bf16& hi, __bf16& lo) {
   hi = (__bf16)v;
   lo = (__bf16)(v - (float)hi);
@@ -275,30 +275,73 @@ __global__ void mfma_prepare(hipmc_glm_hmc_args a) {
   ((__bf16*)a.ws_b)[(size_t)a.n_chains * kMD + i] = lo;
 }
 
-// Sum of the split-N partial gradients of chain c at slot k, plus prior.
+// Element e of chain c: the split-N partial gradients added in split order,
+// plus the prior.  The adds form a serial chain, the loads do not: kU of them
+// are in flight at a time (a few chains take up to N / 32 splits, whose
+// partial sums come from the other XCDs through memory).
 __device__ inline float reduce_grad(const hipmc_glm_hmc_args& a, int c, int e,
                                     float q, float inv_ps2) {
+  constexpr int kU = 32;
+  const float* g = a.ws_g + (size_t)c * kMD + e;
+  const size_t stride = (size_t)a.n_chains * kMD;
+  const int n = a.n_split;
   float s = 0.f;
-  for (int sp = 0; sp < a.n_split; ++sp)
-    s += a.ws_g[((size_t)sp * a.n_chains + c) * kMD + e];
+  int sp = 0;
+  for (; sp + kU <= n; sp += kU) {
+    float v[kU];
+#pragma unroll
+    for (int u = 0; u < kU; ++u) v[u] = g[(size_t)(sp + u) * stride];
+#pragma unroll
+    for (int u = 0; u < kU; ++u) s += v[u];
+  }
+  for (; sp + 8 <= n; sp += 8) {
+    float v[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) v[u] = g[(size_t)(sp + u) * stride];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) s += v[u];
+  }
+  for (; sp < n; ++sp) s += g[(size_t)sp * stride];
   return s - q * inv_ps2;
 }
 
-__device__ inline double reduce_ll(const hipmc_glm_hmc_args& a, int c) {
+// The splits' partial log-likelihoods added in split order (one wave; 64
+// splits are loaded at once, one per lane).
+__device__ inline double reduce_ll(const hipmc_glm_hmc_args& a, int c,
+                                   int lane) {
   double s = 0.0;
-  for (int sp = 0; sp < a.n_split; ++sp) s += (double)a.ws_ll[(size_t)sp * a.n_chains + c];
+  for (int sp = 0; sp < a.n_split; sp += 64) {
+    const int m = a.n_split - sp < 64 ? a.n_split - sp : 64;
+    const float v =
+        lane < m ? a.ws_ll[(size_t)(sp + lane) * a.n_chains + c] : 0.f;
+    for (int l = 0; l < m; ++l) s += (double)readlane_f(v, l);
+  }
   return s;
+}
+
+// Wave 0's share of a block sum: elements lane, 64 + lane, 128 + lane and
+// 192 + lane of v in that order, then over the lanes.
+__device__ inline double element_sum(const double* v, int lane) {
+  return wave_sum(((v[lane] + v[64 + lane]) + v[128 + lane]) + v[192 + lane]);
 }
 
 // mode 0: start of iteration `it` (momentum draw, first half kick, first
 // drift); mode 1: after a gradient of a middle leapfrog step (kick, drift);
 // mode 2: after the last gradient (kick, un-kick, MH accept); mode 3:
 // bootstrap (tlp and grad of the state).
-__global__ void __launch_bounds__(256) mfma_chain_step(hipmc_glm_hmc_args a,
-                                                        int mode, int it) {
-  const int lane = threadIdx.x & 63;
-  const int c = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
-  if (c >= a.n_chains) return;
+// Bound by reading the partial gradients [n_split, chains, 256]: few chains
+// come with many splits, so a thread holds one element (four waves a chain)
+// with up to 32 loads in flight.  Against one wave a chain with dependent
+// loads, us per launch: 64 chains x 256 splits 228 -> 7.1 (17 MB, 2.4 TB/s);
+// 4096 chains x 8 splits 15.1 -> 12.9.  The sums' order is the same.
+__global__ void __launch_bounds__(kMD) mfma_chain_step(hipmc_glm_hmc_args a,
+                                                       int mode, int it) {
+  __shared__ double red[2][kMD];
+  __shared__ double sums[2];
+  const int e = threadIdx.x;
+  const int lane = e & 63;
+  const bool first = e < 64;  // wave 0 does the chain's scalar work
+  const int c = blockIdx.x;
   const float ps = (float)a.prior_scale;
   const float inv_ps = 1.f / ps;
   const float inv_ps2 = inv_ps * inv_ps;
@@ -307,98 +350,96 @@ __global__ void __launch_bounds__(256) mfma_chain_step(hipmc_glm_hmc_args a,
   float* p = a.ws_p + row;
   __bf16* bh = (__bf16*)a.ws_b + row;
   __bf16* bl = (__bf16*)a.ws_b + (size_t)a.n_chains * kMD + row;
-  const float eps = mfma_step_size(a, c);
-  const float half = 0.5f * eps;
   if (mode == 3) {
-    double lp = 0.0;
-    for (int k = 0; k < 4; ++k) {
-      const int e = k * 64 + lane;
-      const float qv = a.state[row + e];
-      a.grad[row + e] = reduce_grad(a, c, e, qv, inv_ps2);
-      const float z = qv * inv_ps;
-      lp += (double)(-0.5f * z * z);
+    const float qv = a.state[row + e];
+    a.grad[row + e] = reduce_grad(a, c, e, qv, inv_ps2);
+    const float z = qv * inv_ps;
+    red[0][e] = (double)(-0.5f * z * z);
+    __syncthreads();
+    if (first) {
+      const double lp = element_sum(red[0], lane);
+      const double ll = reduce_ll(a, c, lane);
+      if (lane == 0)
+        a.tlp[c] = (float)(lp + ll +
+                           kMD * (-0.9189385332046727 - log((double)ps)));
     }
-    lp = wave_sum(lp);
-    if (lane == 0)
-      a.tlp[c] = (float)(lp + reduce_ll(a, c) +
-                         kMD * (-0.9189385332046727 - log((double)ps)));
     return;
   }
+  const float eps = mfma_step_size(a, c);
+  const float half = 0.5f * eps;
   const Seed sd = mfma_iter_seed(a, it);
   if (mode == 0) {
     const Seed prop = split(sd, 0);
-    double ke = 0.0;
-    for (int k = 0; k < 4; ++k) {
-      const int e = k * 64 + lane;
-      const U4 w = philox(U4{(uint32_t)(e >> 2), (uint32_t)c, a.key,
-                             kPurposeMomentum},
-                          prop.k0, prop.k1);
-      const bool hi_pair = (e & 2) != 0;
-      double n0, n1;
-      box_muller(hi_pair ? w.z : w.x, hi_pair ? w.w : w.y, n0, n1);
-      const float pv0 = (float)((e & 1) ? n1 : n0);
-      ke += (double)pv0 * (double)pv0;
-      float pv = pv0 + half * a.grad[row + e];
-      const float qv = a.state[row + e] + eps * pv;
-      p[e] = pv;
-      q[e] = qv;
-      __bf16 hi, lo;
-      split_bf16(qv, hi, lo);
-      bh[e] = hi;
-      bl[e] = lo;
+    const U4 w = philox(U4{(uint32_t)(e >> 2), (uint32_t)c, a.key,
+                           kPurposeMomentum},
+                        prop.k0, prop.k1);
+    const bool hi_pair = (e & 2) != 0;
+    double n0, n1;
+    box_muller(hi_pair ? w.z : w.x, hi_pair ? w.w : w.y, n0, n1);
+    const float pv0 = (float)((e & 1) ? n1 : n0);
+    const float pv = pv0 + half * a.grad[row + e];
+    const float qv = a.state[row + e] + eps * pv;
+    p[e] = pv;
+    q[e] = qv;
+    __bf16 hi, lo;
+    split_bf16(qv, hi, lo);
+    bh[e] = hi;
+    bl[e] = lo;
+    red[0][e] = (double)pv0 * (double)pv0;
+    __syncthreads();
+    if (first) {
+      const double ke = element_sum(red[0], lane);
+      if (lane == 0) a.ws_ke0[c] = 0.5 * ke;
     }
-    ke = wave_sum(ke);
-    if (lane == 0) a.ws_ke0[c] = 0.5 * ke;
     return;
   }
+  const float qv = q[e];
+  const float gv = reduce_grad(a, c, e, qv, inv_ps2);
   if (mode == 1) {
-    for (int k = 0; k < 4; ++k) {
-      const int e = k * 64 + lane;
-      const float gv = reduce_grad(a, c, e, q[e], inv_ps2);
-      const float pv = p[e] + eps * gv;
-      const float qv = q[e] + eps * pv;
-      p[e] = pv;
-      q[e] = qv;
-      __bf16 hi, lo;
-      split_bf16(qv, hi, lo);
-      bh[e] = hi;
-      bl[e] = lo;
-    }
+    const float pv = p[e] + eps * gv;
+    const float qn = qv + eps * pv;
+    p[e] = pv;
+    q[e] = qn;
+    __bf16 hi, lo;
+    split_bf16(qn, hi, lo);
+    bh[e] = hi;
+    bl[e] = lo;
     return;
   }
   // mode 2: last kick, un-kick, kinetic energy, log-prob, MH accept
-  float gv[4], qv[4];
-  double ke = 0.0, lp = 0.0;
-  for (int k = 0; k < 4; ++k) {
-    const int e = k * 64 + lane;
-    qv[k] = q[e];
-    gv[k] = reduce_grad(a, c, e, qv[k], inv_ps2);
-    float pv = p[e] + eps * gv[k];
-    pv = pv - half * gv[k];
-    ke += (double)pv * (double)pv;
-    const float z = qv[k] * inv_ps;
-    lp += (double)(-0.5f * z * z);
+  float pv = p[e] + eps * gv;
+  pv = pv - half * gv;
+  const float z = qv * inv_ps;
+  red[0][e] = (double)pv * (double)pv;
+  red[1][e] = (double)(-0.5f * z * z);
+  __syncthreads();
+  if (first) {
+    const double ke = element_sum(red[0], lane);
+    const double lp = element_sum(red[1], lane);
+    const double ll = reduce_ll(a, c, lane);
+    const double t1 = lp + ll +
+                      kMD * (-0.9189385332046727 - log((double)ps));
+    const double t0 = (double)a.tlp[c];
+    double corr = a.ws_ke0[c] - 0.5 * ke;
+    if (!__builtin_isfinite(corr)) corr = -__builtin_inf();
+    double lar = (t1 - t0) + corr;
+    if (!__builtin_isfinite(lar)) lar = -__builtin_inf();
+    if (lane == 0) {
+      sums[0] = t1;
+      sums[1] = lar;
+    }
   }
-  wave_sum2(ke, lp, ke, lp);
-  const double t1 = lp + reduce_ll(a, c) +
-                    kMD * (-0.9189385332046727 - log((double)ps));
-  const double t0 = (double)a.tlp[c];
-  double corr = a.ws_ke0[c] - 0.5 * ke;
-  if (!__builtin_isfinite(corr)) corr = -__builtin_inf();
-  double lar = (t1 - t0) + corr;
-  if (!__builtin_isfinite(lar)) lar = -__builtin_inf();
+  __syncthreads();
+  const double t1 = sums[0], lar = sums[1];
   const Seed acc = split(sd, 1);
   const U4 uw = philox(U4{0u, (uint32_t)c, a.key, kPurposeMHAccept}, acc.k0,
                        acc.k1);
   const bool accept = log((double)uniform_from<float>(uw.x, uw.y)) < lar;
   if (accept) {
-    for (int k = 0; k < 4; ++k) {
-      const int e = k * 64 + lane;
-      a.state[row + e] = qv[k];
-      a.grad[row + e] = gv[k];
-    }
+    a.state[row + e] = qv;
+    a.grad[row + e] = gv;
   }
-  if (lane == 0) {
+  if (e == 0) {
     if (accept) a.tlp[c] = (float)t1;
     const size_t o = (size_t)it * a.n_chains + c;
     if (a.out_log_accept_ratio) a.out_log_accept_ratio[o] = (float)lar;
@@ -409,10 +450,7 @@ __global__ void __launch_bounds__(256) mfma_chain_step(hipmc_glm_hmc_args a,
     const int every = a.trace_every > 0 ? a.trace_every : 1;
     if (gi >= 0 && gi % every == 0 && gi / every < a.n_trace) {
       float* tr = a.trace_state + ((size_t)(gi / every) * a.n_chains + c) * kMD;
-      for (int k = 0; k < 4; ++k) {
-        const int e = k * 64 + lane;
-        tr[e] = a.state[row + e];
-      }
+      tr[e] = accept ? qv : a.state[row + e];
     }
   }
 }

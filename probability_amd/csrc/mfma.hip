@@ -79,7 +79,7 @@ int launch_glm_hmc(const hipmc_glm_hmc_args* a, hipStream_t s) {
   // then serves 8 waves), else 64
   const bool wide = a->n_chains % (2 * kMChains) == 0;
   const dim3 ggrid(a->n_chains / (wide ? 2 * kMChains : kMChains), n_split);
-  const dim3 cgrid((a->n_chains + 3) / 4);
+  const dim3 cgrid(a->n_chains);
   auto grad = [&](bool ll) {
     const __bf16* bh = (const __bf16*)a->ws_b;
     const __bf16* bl = bh + (size_t)a->n_chains * kMD;
@@ -100,15 +100,15 @@ int launch_glm_hmc(const hipmc_glm_hmc_args* a, hipStream_t s) {
     hipLaunchKernelGGL(mfma_prepare, dim3(blocks_for(ne, 256)), dim3(256), 0,
                        s, *a);
     grad(true);
-    hipLaunchKernelGGL(mfma_chain_step, cgrid, dim3(256), 0, s, *a, 3, 0);
+    hipLaunchKernelGGL(mfma_chain_step, cgrid, dim3(kMD), 0, s, *a, 3, 0);
     return hip_check(hipGetLastError(), "glm_hmc bootstrap launch");
   }
   for (int it = 0; it < a->n_iters; ++it) {
-    hipLaunchKernelGGL(mfma_chain_step, cgrid, dim3(256), 0, s, *a, 0, it);
+    hipLaunchKernelGGL(mfma_chain_step, cgrid, dim3(kMD), 0, s, *a, 0, it);
     for (int st = 0; st < a->num_leapfrog_steps; ++st) {
       const bool last = st + 1 == a->num_leapfrog_steps;
       grad(last);
-      hipLaunchKernelGGL(mfma_chain_step, cgrid, dim3(256), 0, s, *a,
+      hipLaunchKernelGGL(mfma_chain_step, cgrid, dim3(kMD), 0, s, *a,
                          last ? 2 : 1, it);
     }
   }
