@@ -503,6 +503,42 @@ int hipmc_draws(int32_t dtype, int32_t kind, const uint32_t seed[2],
                 int32_t problem, int32_t n_chains, int32_t dim, int32_t depth,
                 int32_t index, void* out, uint8_t* out_aux, uint64_t stream);
 
+/*
+ * Cross-chain effective sample size of draws x (dtype; element (t, c, d) at
+ * t * stride_n + c * stride_chain + d * stride_dim, strides in elements), all
+ * in float64: per dimension d the autocovariance averaged over the chains, its
+ * autocorrelation against the between-chain variance, and
+ * chains n / (-1 + 2 sum_k (n - k) / n rho_k), the sum ending before the first
+ * rho_k below `threshold` if truncate is non-zero.  2 <= chains,
+ * 1 <= n <= 4096.  out: float64 [dims].  Workspaces: ws_rows dtype
+ * [dims, chains, n]; ws_means float64 [dims, chains]; ws_power float64
+ * [blocks, dims, m] with m the power of two >= max(2 n, 16).  `blocks`: the
+ * blocks that share a dimension's chains.  Replaces effective_sample_size
+ * with cross_chain_dims (mcmc/diagnostic.py:203-336).
+ */
+int hipmc_effective_sample_size(int32_t dtype, int64_t n, int64_t chains,
+                                int64_t dims, int64_t stride_n,
+                                int64_t stride_chain, int64_t stride_dim,
+                                const void* x, int32_t truncate,
+                                double threshold, int32_t blocks, void* ws_rows,
+                                double* ws_means, double* ws_power, double* out,
+                                uint64_t stream);
+
+/*
+ * R-hat of draws x (as above), in float64; split != 0 takes each chain's two
+ * halves of n / 2 draws as chains (an odd last draw is left out).  At least
+ * two draws per half.  out: float64 [dims]; ws_sums: float64
+ * [chunks, split ? 2 : 1, 2, chains * dims], `chunks` the time chunks whose
+ * partial sums are added in order.  Replaces potential_scale_reduction
+ * (mcmc/diagnostic.py:476-568).
+ */
+int hipmc_potential_scale_reduction(int32_t dtype, int64_t n, int64_t chains,
+                                    int64_t dims, int64_t stride_n,
+                                    int64_t stride_chain, int64_t stride_dim,
+                                    const void* x, int32_t split,
+                                    int32_t chunks, double* ws_sums,
+                                    double* out, uint64_t stream);
+
 #ifdef __cplusplus
 }
 #endif

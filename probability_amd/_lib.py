@@ -31,7 +31,8 @@ EXPORTED_SYMBOLS = (
     'hipmc_leapfrog_run', 'hipmc_nuts_run', 'hipmc_target_eval',
     'hipmc_da_update', 'hipmc_simple_step_update', 'hipmc_mh_accept',
     'hipmc_bijector', 'hipmc_draws', 'hipmc_moments_update',
-    'hipmc_variance_update', 'hipmc_glm_hmc_run_noalloc')
+    'hipmc_variance_update', 'hipmc_glm_hmc_run_noalloc',
+    'hipmc_effective_sample_size', 'hipmc_potential_scale_reduction')
 
 _vp = ctypes.c_void_p
 _i32 = ctypes.c_int32
@@ -143,6 +144,12 @@ def lib():
                                     _u64]
       l.hipmc_moments_update.argtypes = [_i32, _i32, _i64, _i64, _i64, _vp,
                                          _f64, _vp, _vp, _vp, _vp, _u64]
+      l.hipmc_effective_sample_size.argtypes = [
+          _i32, _i64, _i64, _i64, _i64, _i64, _i64, _vp, _i32, _f64, _i32, _vp,
+          _vp, _vp, _vp, _u64]
+      l.hipmc_potential_scale_reduction.argtypes = [
+          _i32, _i64, _i64, _i64, _i64, _i64, _i64, _vp, _i32, _i32, _vp, _vp,
+          _u64]
       l.hipmc_bijector.argtypes = [_i32, _vp, _vp, _i32, _i32, _i32, _i32,
                                    _vp, _vp, _u64]
       l.hipmc_draws.argtypes = [_i32, _i32, _vp, _i32, _i32, _i32, _i32, _i32,

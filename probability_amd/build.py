@@ -1,8 +1,8 @@
 """Builds libhipmc.so in-tree with hipcc for gfx950.
 
 The library is linked from several objects compiled in parallel: the ABI
-and small kernels (hipmc.hip), the BF16 MFMA path (mfma.hip) and the
-sampling kernels, one object per (kernel group, dtype, target family) from
+and small kernels (hipmc.hip), the BF16 MFMA path (mfma.hip), the
+convergence diagnostics (diagnostic.hip) and the sampling kernels, one object per (kernel group, dtype, target family) from
 inst.hip.
 
 Usage: python -m probability_amd.build   (or probability_amd.build.build()).
@@ -31,7 +31,8 @@ _FAMILIES = {'hier': 0, 'glm': 1, 'test': 2}
 
 def objects():
   """(object name, source, extra defines) of every object of the library."""
-  out = [('hipmc', 'hipmc.hip', []), ('mfma', 'mfma.hip', [])]
+  out = [('hipmc', 'hipmc.hip', []), ('mfma', 'mfma.hip', []),
+         ('diagnostic', 'diagnostic.hip', [])]
   for group, nuts in (('nuts', 1), ('hmc', 0)):
     for t in ('float', 'double'):
       for fam, code in _FAMILIES.items():

@@ -1,0 +1,664 @@
+// Convergence diagnostics of a finished run: cross-chain effective sample
+// size and (split) R-hat of draws [n, chains, dims] in float32 or float64,
+// computed in float64 (mcmc/diagnostic.py:38-568, stats/sample_stats.py:
+// 44-216).
+//
+// The effective sample size needs, per dimension, the autocovariance at
+// every lag averaged over the chains:
+//   ess_transpose  draws -> one contiguous row per (dimension, chain)
+//   ess_power      per (dimension, block of chains): chains are centred and
+//                  transformed two at a time, z = x1 + i x2, zero-padded to
+//                  m = 2^ceil(log2 2n) points in LDS, and |Z|^2 is added up.
+//                  The real part of the inverse transform of |Z|^2 is the sum
+//                  of the two autocorrelations, so neither the two spectra
+//                  nor the bit-reversed order of the in-place transform ever
+//                  have to be taken apart.
+//   ess_finish     per dimension: one inverse transform of the chains' summed
+//                  power, the variance of the chain means, the
+//                  autocorrelation, its truncation and the sum.
+// As float64 library operations (two transforms of every series, complex
+// products, copies, a cumulative sum: some forty passes over 65 to 270 MB at
+// 1000 x 64 x 127 float32 draws) ESS and split R-hat took 1446 us together;
+// these kernels take 82 (ess_power 36, ess_transpose 20 at 3.2 TB/s,
+// ess_finish 13, the R-hat kernels 17).
+#include <hip/hip_runtime.h>
+
+#include <cmath>
+#include <string>
+
+#include "../../include/hipmc.h"
+#include "common.h"
+#include "runtime.h"
+
+namespace hipmc {
+namespace {
+
+struct Cplx {
+  double re, im;
+};
+__device__ inline Cplx operator+(Cplx a, Cplx b) {
+  return Cplx{a.re + b.re, a.im + b.im};
+}
+__device__ inline Cplx operator-(Cplx a, Cplx b) {
+  return Cplx{a.re - b.re, a.im - b.im};
+}
+__device__ inline Cplx operator*(Cplx a, Cplx b) {
+  return Cplx{a.re * b.re - a.im * b.im, a.re * b.im + a.im * b.re};
+}
+// a times -i (forward) or i (inverse)
+template <bool INV>
+__device__ inline Cplx quarter(Cplx a) {
+  return INV ? Cplx{-a.im, a.re} : Cplx{a.im, -a.re};
+}
+
+// Unnormalised transforms of 2, 4 and 8 points, results in natural order.
+__device__ inline void dft2(Cplx& a, Cplx& b) {
+  const Cplx s = a + b;
+  b = a - b;
+  a = s;
+}
+template <bool INV>
+__device__ inline void dft4(Cplx& a, Cplx& b, Cplx& c, Cplx& d) {
+  const Cplx t0 = a + c, t1 = a - c, t2 = b + d, t3 = quarter<INV>(b - d);
+  a = t0 + t2;
+  c = t0 - t2;
+  b = t1 + t3;
+  d = t1 - t3;
+}
+template <bool INV>
+__device__ inline void dft8(Cplx (&v)[8]) {
+  dft4<INV>(v[0], v[2], v[4], v[6]);  // even terms, results in 0 2 4 6
+  dft4<INV>(v[1], v[3], v[5], v[7]);  // odd terms, results in 1 3 5 7
+  const double h = 0.70710678118654752440;
+  const double s = INV ? h : -h;
+  v[3] = v[3] * Cplx{h, s};
+  v[5] = quarter<INV>(v[5]);
+  v[7] = v[7] * Cplx{-h, s};
+  const Cplx e0 = v[0], e1 = v[2], e2 = v[4], e3 = v[6];
+  const Cplx o0 = v[1], o1 = v[3], o2 = v[5], o3 = v[7];
+  v[0] = e0 + o0;
+  v[1] = e1 + o1;
+  v[2] = e2 + o2;
+  v[3] = e3 + o3;
+  v[4] = e0 - o0;
+  v[5] = e1 - o1;
+  v[6] = e2 - o2;
+  v[7] = e3 - o3;
+}
+
+// In-place transform of m = 2^L points by m / 8 threads, one radix-8
+// butterfly each per pass: L / 3 radix-8 passes (decimation in frequency),
+// the last of which, or the remaining one or two levels, works on the
+// thread's eight consecutive points.  Pass i takes blocks of m / 8^i points.
+template <int L>
+struct Fft {
+  static constexpr int M = 1 << L;
+  static constexpr int kLive = M / 8;                    // threads with work
+  static constexpr int kThreads = kLive < 64 ? 64 : kLive;
+  static constexpr int kPasses = (L - 1) / 3;            // twiddled passes
+  static constexpr int kLast = L - 3 * kPasses;          // levels of the last
+  // One unused element after every eight keeps the last pass (eight
+  // consecutive points a thread) and the passes of short blocks off each
+  // other's LDS banks.
+  static constexpr int kElems = M + M / 8;
+  static constexpr size_t kBytes = 2 * (size_t)kElems * sizeof(double);
+  static __device__ int at(int i) { return i + (i >> 3); }
+  // points of one eighth of a block of pass p
+  static constexpr int eighth(int p) { return M >> (3 * (p + 1)); }
+
+  // exp(-2 pi i r / block) of this thread's butterfly in every pass
+  static __device__ void twiddles(int tid, Cplx (&w)[kPasses]) {
+#pragma unroll
+    for (int p = 0; p < kPasses; ++p) {
+      const int q = eighth(p);
+      const int r = tid & (q - 1);
+      double s, c;
+      sincospi(-2.0 * (double)r / (double)(8 * q), &s, &c);
+      w[p] = Cplx{c, s};
+    }
+  }
+  static __device__ int base(int tid, int p) {
+    const int q = eighth(p);
+    return (tid & ~(q - 1)) * 8 + (tid & (q - 1));
+  }
+  // v[u] *= w^u (forward) or conj(w)^u (inverse)
+  template <bool INV>
+  static __device__ void turn(Cplx (&v)[8], Cplx w) {
+    if (INV) w.im = -w.im;
+    const Cplx w2 = w * w, w3 = w2 * w, w4 = w2 * w2;
+    v[1] = v[1] * w;
+    v[2] = v[2] * w2;
+    v[3] = v[3] * w3;
+    v[4] = v[4] * w4;
+    v[5] = v[5] * (w4 * w);
+    v[6] = v[6] * (w4 * w2);
+    v[7] = v[7] * (w4 * w3);
+  }
+  template <bool INV>
+  static __device__ void last(Cplx (&v)[8]) {
+    if (kLast == 1) {
+#pragma unroll
+      for (int u = 0; u < 8; u += 2) dft2(v[u], v[u + 1]);
+    } else if (kLast == 2) {
+#pragma unroll
+      for (int u = 0; u < 8; u += 4)
+        dft4<INV>(v[u], v[u + 1], v[u + 2], v[u + 3]);
+    } else {
+      dft8<INV>(v);
+    }
+  }
+  static __device__ void put(double* re, double* im, int i0, int step,
+                             const Cplx (&v)[8]) {
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const int k = at(i0 + u * step);
+      re[k] = v[u].re;
+      im[k] = v[u].im;
+    }
+  }
+  static __device__ void get(const double* re, const double* im, int i0,
+                             int step, Cplx (&v)[8]) {
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const int k = at(i0 + u * step);
+      v[u] = Cplx{re[k], im[k]};
+    }
+  }
+  // v: points tid + u * M / 8 on entry; on return the thread's eight
+  // consecutive results of the transform's own order.  Every thread of the
+  // block calls it (it holds barriers); threads past kLive do no work.
+  static __device__ void forward(double* re, double* im, int tid,
+                                 const Cplx (&w)[kPasses], Cplx (&v)[8]) {
+    const bool live = tid < kLive;
+#pragma unroll
+    for (int p = 0; p < kPasses; ++p) {
+      if (live) {
+        if (p > 0) get(re, im, base(tid, p), eighth(p), v);
+        dft8<false>(v);
+        turn<false>(v, w[p]);
+        put(re, im, base(tid, p), eighth(p), v);
+      }
+      __syncthreads();
+    }
+    if (live) {
+      get(re, im, 8 * tid, 1, v);
+      last<false>(v);
+    }
+  }
+  // The inverse of forward() times M.
+  static __device__ void inverse(double* re, double* im, int tid,
+                                 const Cplx (&w)[kPasses], Cplx (&v)[8]) {
+    const bool live = tid < kLive;
+    if (live) {
+      last<true>(v);
+      put(re, im, 8 * tid, 1, v);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int p = kPasses - 1; p >= 0; --p) {
+      if (live) {
+        get(re, im, base(tid, p), eighth(p), v);
+        turn<true>(v, w[p]);
+        dft8<true>(v);
+        if (p > 0) put(re, im, base(tid, p), eighth(p), v);
+      }
+      __syncthreads();
+    }
+  }
+};
+
+// Sum over the block's threads of a and b, given to every thread; `red` holds
+// 2 doubles per wave.  Ends with the buffer free for the next call.
+__device__ inline void block_sum2(double& a, double& b, double* red) {
+  const int wave = threadIdx.x >> 6, waves = (blockDim.x + 63) >> 6;
+  double sa, sb;
+  wave_sum2(a, b, sa, sb);
+  if (lane_id() == 0) {
+    red[2 * wave] = sa;
+    red[2 * wave + 1] = sb;
+  }
+  __syncthreads();
+  a = 0.0;
+  b = 0.0;
+  for (int w = 0; w < waves; ++w) {
+    a += red[2 * w];
+    b += red[2 * w + 1];
+  }
+  __syncthreads();
+}
+
+// draws x[t * sn + c * sc + d * sd] -> out[(d * chains + c) * n + t].  Tiles of
+// 64 draws x 64 series (series s = c * dims + d, so that consecutive lanes
+// read consecutive dimensions) turned over in LDS.
+template <typename T>
+__global__ void __launch_bounds__(256)
+    ess_transpose(const T* __restrict__ x, int n, int chains, int dims,
+                  int64_t sn, int64_t sc, int64_t sd, T* __restrict__ out) {
+  __shared__ T tile[64][65];
+  const int64_t series = (int64_t)chains * dims;
+  const int lane = threadIdx.x & 63, part = threadIdx.x >> 6;
+  const int64_t s0 = (int64_t)blockIdx.x * 64;
+  const int t0 = blockIdx.y * 64;
+  {
+    const int64_t s = s0 + lane;
+    if (s < series) {
+      const int64_t c = s / dims, d = s - c * dims;
+      const T* src = x + c * sc + d * sd;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        const int t = t0 + part + 4 * i;
+        if (t < n) tile[part + 4 * i][lane] = src[(int64_t)t * sn];
+      }
+    }
+  }
+  __syncthreads();
+  const int t = t0 + lane;
+  if (t >= n) return;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    const int64_t s = s0 + part + 4 * i;
+    if (s >= series) return;
+    const int64_t c = s / dims, d = s - c * dims;
+    out[(d * chains + c) * n + t] = tile[lane][part + 4 * i];
+  }
+}
+
+// Block (d, y): chain pairs [y * per, (y + 1) * per) of dimension d.  Writes
+// the chains' means [dims, chains] and this block's summed power
+// [blocks y, dims, m].
+// Bound by the serial passes of a pair (four at 2048 points, 192 KiB through
+// LDS) at two blocks a CU: the butterflies take 189 registers; held to 168 for
+// three blocks a CU they spill, 36 -> 43 us at 1000 x 64 x 127.
+template <typename T, int L>
+__global__ void __launch_bounds__(Fft<L>::kThreads)
+    ess_power(const T* __restrict__ rows, int n, int chains, int dims, int per,
+              double* __restrict__ means, double* __restrict__ power) {
+  using F = Fft<L>;
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  __shared__ double red[2 * (F::kThreads / 64)];
+  double* re = (double*)smem_raw;
+  double* im = re + F::kElems;
+  const int tid = threadIdx.x;
+  const int d = blockIdx.x;
+  Cplx w[F::kPasses];
+  F::twiddles(tid, w);
+  double acc[8];
+#pragma unroll
+  for (int u = 0; u < 8; ++u) acc[u] = 0.0;
+  const int pairs = (chains + 1) >> 1;
+  const int p1 = min(pairs, (int)(blockIdx.y + 1) * per);
+  // the thread's draws of a pair (t = tid + u m / 8; n <= m / 2): the next
+  // pair's are loaded while the current one is transformed
+  T a1[4], a2[4];
+  auto load = [&](int p) {
+    const int c = 2 * p;
+    const T* x1 = rows + ((size_t)d * chains + c) * n;
+    const T* x2 = c + 1 < chains ? x1 + n : x1;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int t = tid + u * (F::M / 8);
+      const bool in = tid < F::kLive && t < n;
+      a1[u] = in ? x1[t] : T(0);
+      a2[u] = in ? x2[t] : T(0);
+    }
+  };
+  const int p0 = blockIdx.y * per;
+  if (p0 < p1) load(p0);
+  for (int p = p0; p < p1; ++p) {
+    const int c = 2 * p;
+    const bool two = c + 1 < chains;
+    double m1 = 0.0, m2 = 0.0;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      m1 += (double)a1[u];
+      m2 += (double)a2[u];
+    }
+    block_sum2(m1, m2, red);
+    m1 /= (double)n;
+    m2 /= (double)n;
+    if (tid == 0) {
+      means[(size_t)d * chains + c] = m1;
+      if (two) means[(size_t)d * chains + c + 1] = m2;
+    }
+    Cplx v[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const int t = tid + u * (F::M / 8);
+      const bool in = tid < F::kLive && u < 4 && t < n;
+      v[u].re = in ? (double)a1[u & 3] - m1 : 0.0;
+      v[u].im = in && two ? (double)a2[u & 3] - m2 : 0.0;
+    }
+    if (p + 1 < p1) load(p + 1);
+    F::forward(re, im, tid, w, v);
+#pragma unroll
+    for (int u = 0; u < 8; ++u) acc[u] += v[u].re * v[u].re + v[u].im * v[u].im;
+    __syncthreads();  // the next pair overwrites the buffer
+  }
+  if (tid < F::kLive) {
+    double* out = power + ((size_t)blockIdx.y * dims + d) * F::M + tid;
+#pragma unroll
+    for (int u = 0; u < 8; ++u) out[u * F::kLive] = acc[u];
+  }
+}
+
+// One block per dimension.  With ac[k] the mean over the chains of the
+// autocovariance at lag k, w = ac[0] and b the variance of the chain means:
+//   rho[k] = 1 - (w - ac[k]) / (w + b),
+//   ess = chains n / (-1 + 2 sum_k (n - k) / n rho[k] keep[k])
+// where keep is 1 before the first rho below `threshold` and 0 from it on
+// (always 1 if truncate is 0).  The terms are multiplied by keep, so a NaN
+// beyond the truncation makes the result NaN as it does in the reference.
+template <int L>
+__global__ void __launch_bounds__(Fft<L>::kThreads)
+    ess_finish(const double* __restrict__ power, int blocks, int n, int chains,
+               int dims, const double* __restrict__ means, int truncate,
+               double threshold, double* __restrict__ out) {
+  using F = Fft<L>;
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  __shared__ double red[2 * (F::kThreads / 64)];
+  __shared__ double lag0;
+  __shared__ int first;
+  double* re = (double*)smem_raw;
+  double* im = re + F::kElems;
+  const int tid = threadIdx.x;
+  const int d = blockIdx.x;
+  Cplx w[F::kPasses];
+  F::twiddles(tid, w);
+  Cplx v[8];
+#pragma unroll
+  for (int u = 0; u < 8; ++u) v[u] = Cplx{0.0, 0.0};
+  if (tid < F::kLive) {
+#pragma unroll 4
+    for (int y = 0; y < blocks; ++y) {
+      const double* src = power + ((size_t)y * dims + d) * F::M + tid;
+#pragma unroll
+      for (int u = 0; u < 8; ++u) v[u].re += src[u * F::kLive];
+    }
+  }
+  if (tid == 0) first = n;
+  F::inverse(re, im, tid, w, v);
+  // v[u].re = M chains (n - k) ac[k] at k = tid + u M / 8
+  double ac[4];
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    const int k = tid + u * (F::M / 8);
+    ac[u] = k < n ? v[u].re / ((double)F::M * (double)chains * (double)(n - k))
+                  : 0.0;
+  }
+  if (tid == 0) lag0 = ac[0];
+  double s = 0.0, q = 0.0;
+  for (int c = tid; c < chains; c += F::kThreads)
+    s += means[(size_t)d * chains + c];
+  block_sum2(s, q, red);  // its barriers also publish lag0 and first
+  const double mu = s / (double)chains;
+  s = 0.0;
+  for (int c = tid; c < chains; c += F::kThreads) {
+    const double e = means[(size_t)d * chains + c] - mu;
+    s += e * e;
+  }
+  block_sum2(s, q, red);
+  const double var = s / (double)(chains - 1);
+  const double w0 = lag0;
+  double rho[4];
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    const int k = tid + u * (F::M / 8);
+    rho[u] = 1.0 - (w0 - ac[u]) / (w0 + var);
+    if (truncate && tid < F::kLive && k < n && rho[u] < threshold)
+      atomicMin(&first, k);
+  }
+  __syncthreads();
+  double total = 0.0;
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    const int k = tid + u * (F::M / 8);
+    if (tid < F::kLive && k < n)
+      total += (double)(n - k) / (double)n * rho[u] * (k < first ? 1.0 : 0.0);
+  }
+  double none = 0.0;
+  block_sum2(total, none, red);
+  if (tid == 0)
+    out[d] = (double)chains * (double)n / (-1.0 + 2.0 * total);
+}
+
+// Sums of (x - x0) and (x - x0)^2 of every series (and half of it, with
+// halves = 2), x0 the first draw of the half: x0 is one of the draws summed,
+// so its distance from the mean is at most sqrt(n) standard deviations and
+// the variance keeps all but a factor n of float64's precision.  Block
+// (64 series) x (4 interleaved time steps), grid y = half, z = time chunk;
+// out [z, half, 2, series].  Bound by HBM (each draw is read once).
+template <typename T>
+__global__ void __launch_bounds__(256)
+    rhat_sums(const T* __restrict__ x, int h, int chains, int dims, int64_t sn,
+              int64_t sc, int64_t sd, int chunk, double* __restrict__ out) {
+  __shared__ double red[2][4][64];
+  const int lane = threadIdx.x & 63, part = threadIdx.x >> 6;
+  const int64_t series = (int64_t)chains * dims;
+  const int64_t s = (int64_t)blockIdx.x * 64 + lane;
+  double a = 0.0, b = 0.0;
+  if (s < series) {
+    const int64_t c = s / dims, d = s - c * dims;
+    const T* src = x + c * sc + d * sd + (int64_t)blockIdx.y * h * sn;
+    const double x0 = (double)src[0];
+    const int t1 = min(h, (int)(blockIdx.z + 1) * chunk);
+#pragma unroll 8
+    for (int t = blockIdx.z * chunk + part; t < t1; t += 4) {
+      const double e = (double)src[(int64_t)t * sn] - x0;
+      a += e;
+      b += e * e;
+    }
+  }
+  red[0][part][lane] = a;
+  red[1][part][lane] = b;
+  __syncthreads();
+  if (part < 2 && s < series)
+    out[(((size_t)blockIdx.z * gridDim.y + blockIdx.y) * 2 + part) * series +
+        s] = ((red[part][0][lane] + red[part][1][lane]) + red[part][2][lane]) +
+             red[part][3][lane];
+}
+
+// One block per dimension: with the mean and unbiased variance of each of the
+// m = halves * chains series of h draws, w the mean of the variances and b
+// the unbiased variance of the means,
+//   s2 = (h - 1) / h w + b,  R-hat = (m + 1) / m s2 / w - (h - 1) / (m h).
+// The first kKeep series of a thread keep their means between the two sums;
+// any others are read again.
+template <typename T>
+__global__ void __launch_bounds__(256)
+    rhat_finish(const double* __restrict__ sums, const T* __restrict__ x, int h,
+                int halves, int chains, int dims, int64_t sn, int64_t sc,
+                int64_t sd, int chunks, double* __restrict__ out) {
+  __shared__ double red[8];
+  constexpr int kKeep = 4;
+  const int d = blockIdx.x;
+  const int tid = threadIdx.x;
+  const int64_t series = (int64_t)chains * dims;
+  const int m = halves * chains;
+  const double hn = (double)h;
+  auto stats = [&](int i, double& mean, double& var) {
+    const int half = i / chains, c = i - half * chains;
+    const int64_t s = (int64_t)c * dims + d;
+    const double x0 = (double)x[c * sc + d * sd + (int64_t)half * h * sn];
+    double a = 0.0, b = 0.0;
+#pragma unroll 8
+    for (int z = 0; z < chunks; ++z) {
+      const double* p = sums + ((size_t)z * halves + half) * 2 * series + s;
+      a += p[0];
+      b += p[series];
+    }
+    mean = x0 + a / hn;
+    var = (b - a * (a / hn)) / (hn - 1.0);
+  };
+  double kept[kKeep];
+  double sm = 0.0, sv = 0.0;
+#pragma unroll
+  for (int u = 0; u < kKeep; ++u) {
+    const int i = tid + 256 * u;
+    double var = 0.0;
+    kept[u] = 0.0;
+    if (i < m) stats(i, kept[u], var);
+    sm += kept[u];
+    sv += var;
+  }
+  for (int i = tid + 256 * kKeep; i < m; i += 256) {
+    double mean, var;
+    stats(i, mean, var);
+    sm += mean;
+    sv += var;
+  }
+  block_sum2(sm, sv, red);
+  const double mu = sm / (double)m, w = sv / (double)m;
+  double sq = 0.0, none = 0.0;
+#pragma unroll
+  for (int u = 0; u < kKeep; ++u)
+    if (tid + 256 * u < m) sq += (kept[u] - mu) * (kept[u] - mu);
+  for (int i = tid + 256 * kKeep; i < m; i += 256) {
+    double mean, var;
+    stats(i, mean, var);
+    sq += (mean - mu) * (mean - mu);
+  }
+  block_sum2(sq, none, red);
+  const double b = sq / ((double)m - 1.0);
+  if (tid == 0) {
+    const double s2 = (hn - 1.0) / hn * w + b;
+    out[d] = ((double)m + 1.0) / (double)m * s2 / w -
+             (hn - 1.0) / ((double)m * hn);
+  }
+}
+
+template <typename F>
+int allow_dynamic_lds(F* kernel, size_t bytes) {
+  if (bytes <= (size_t)kMaxLdsPerBlock) return HIPMC_OK;
+  return hip_check(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
+                                       hipFuncAttributeMaxDynamicSharedMemorySize,
+                                       (int)bytes),
+                   "hipFuncSetAttribute(max dynamic LDS)");
+}
+
+template <typename T, int L>
+int ess_launch(const T* rows, int n, int chains, int dims, int blocks,
+               int truncate, double threshold, double* means, double* power,
+               double* out, hipStream_t s) {
+  using F = Fft<L>;
+  int rc = allow_dynamic_lds(&ess_power<T, L>, F::kBytes);
+  if (rc != HIPMC_OK) return rc;
+  rc = allow_dynamic_lds(&ess_finish<L>, F::kBytes);
+  if (rc != HIPMC_OK) return rc;
+  const int pairs = (chains + 1) / 2;
+  const int per = (pairs + blocks - 1) / blocks;
+  hipLaunchKernelGGL((ess_power<T, L>), dim3(dims, blocks), dim3(F::kThreads),
+                     F::kBytes, s, rows, n, chains, dims, per, means, power);
+  hipLaunchKernelGGL((ess_finish<L>), dim3(dims), dim3(F::kThreads), F::kBytes,
+                     s, power, blocks, n, chains, dims, means, truncate,
+                     threshold, out);
+  return hip_check(hipGetLastError(), "ess launch");
+}
+
+template <typename T>
+int ess_run(int n, int chains, int dims, int64_t sn, int64_t sc, int64_t sd,
+            const T* x, int truncate, double threshold, int blocks, T* rows,
+            double* means, double* power, double* out, hipStream_t s) {
+  const int64_t series = (int64_t)chains * dims;
+  hipLaunchKernelGGL(ess_transpose<T>,
+                     dim3((unsigned)((series + 63) / 64), (n + 63) / 64),
+                     dim3(256), 0, s, x, n, chains, dims, sn, sc, sd, rows);
+  int l = 4;
+  while ((1 << l) < 2 * n) ++l;
+  switch (l) {
+#define HIPMC_ESS(LL)                                                       \
+  case LL:                                                                  \
+    return ess_launch<T, LL>(rows, n, chains, dims, blocks, truncate,       \
+                             threshold, means, power, out, s);
+    HIPMC_ESS(4) HIPMC_ESS(5) HIPMC_ESS(6) HIPMC_ESS(7) HIPMC_ESS(8)
+    HIPMC_ESS(9) HIPMC_ESS(10) HIPMC_ESS(11) HIPMC_ESS(12) HIPMC_ESS(13)
+#undef HIPMC_ESS
+  }
+  return fail(HIPMC_E_UNSUPPORTED, "ess: more than 4096 draws");
+}
+
+template <typename T>
+int rhat_run(int h, int halves, int chains, int dims, int64_t sn, int64_t sc,
+             int64_t sd, const T* x, int chunks, double* sums, double* out,
+             hipStream_t s) {
+  const int64_t series = (int64_t)chains * dims;
+  const int chunk = (h + chunks - 1) / chunks;
+  hipLaunchKernelGGL(rhat_sums<T>,
+                     dim3((unsigned)((series + 63) / 64), halves, chunks),
+                     dim3(256), 0, s, x, h, chains, dims, sn, sc, sd, chunk,
+                     sums);
+  hipLaunchKernelGGL(rhat_finish<T>, dim3(dims), dim3(256), 0, s, sums, x, h,
+                     halves, chains, dims, sn, sc, sd, chunks, out);
+  return hip_check(hipGetLastError(), "rhat launch");
+}
+
+int check_draws(const char* what, int32_t dtype, int64_t n, int64_t chains,
+                int64_t dims) {
+  if (dtype != HIPMC_F32 && dtype != HIPMC_F64)
+    return fail(HIPMC_E_INVALID, std::string(what) + ": bad dtype");
+  if (n < 1 || chains < 1 || dims < 1)
+    return fail(HIPMC_E_INVALID,
+                std::string(what) + ": draws, chains and dims must be >= 1");
+  if (chains > (1 << 30) || dims > (1 << 30) || chains * dims > (1LL << 36))
+    return fail(HIPMC_E_UNSUPPORTED, std::string(what) + ": too many series");
+  return HIPMC_OK;
+}
+
+}  // namespace
+}  // namespace hipmc
+
+using namespace hipmc;
+
+extern "C" {
+
+int hipmc_effective_sample_size(int32_t dtype, int64_t n, int64_t chains,
+                                int64_t dims, int64_t stride_n,
+                                int64_t stride_chain, int64_t stride_dim,
+                                const void* x, int32_t truncate,
+                                double threshold, int32_t blocks, void* ws_rows,
+                                double* ws_means, double* ws_power, double* out,
+                                uint64_t stream) {
+  const int rc = check_draws("ess", dtype, n, chains, dims);
+  if (rc) return rc;
+  if (!x || !ws_rows || !ws_means || !ws_power || !out)
+    return fail(HIPMC_E_INVALID, "ess: NULL argument");
+  if (chains < 2) return fail(HIPMC_E_INVALID, "ess: needs > 1 chain");
+  if (n > 4096) return fail(HIPMC_E_UNSUPPORTED, "ess: more than 4096 draws");
+  if (blocks < 1 || blocks > 65535)
+    return fail(HIPMC_E_INVALID, "ess: blocks must be in [1, 65535]");
+  hipStream_t s = as_stream(stream);
+  if (dtype == HIPMC_F32)
+    return ess_run((int)n, (int)chains, (int)dims, stride_n, stride_chain,
+                   stride_dim, (const float*)x, truncate, threshold, blocks,
+                   (float*)ws_rows, ws_means, ws_power, out, s);
+  return ess_run((int)n, (int)chains, (int)dims, stride_n, stride_chain,
+                 stride_dim, (const double*)x, truncate, threshold, blocks,
+                 (double*)ws_rows, ws_means, ws_power, out, s);
+}
+
+int hipmc_potential_scale_reduction(int32_t dtype, int64_t n, int64_t chains,
+                                    int64_t dims, int64_t stride_n,
+                                    int64_t stride_chain, int64_t stride_dim,
+                                    const void* x, int32_t split,
+                                    int32_t chunks, double* ws_sums,
+                                    double* out, uint64_t stream) {
+  const int rc = check_draws("rhat", dtype, n, chains, dims);
+  if (rc) return rc;
+  if (!x || !ws_sums || !out)
+    return fail(HIPMC_E_INVALID, "rhat: NULL argument");
+  const int halves = split ? 2 : 1;
+  if (n / halves < 2 || n > (1 << 30))
+    return fail(HIPMC_E_INVALID, "rhat: needs 2 to 2^30 draws per half");
+  if (chains > (1 << 29))
+    return fail(HIPMC_E_UNSUPPORTED, "rhat: too many chains");
+  if (chunks < 1 || chunks > 65535)
+    return fail(HIPMC_E_INVALID, "rhat: chunks must be in [1, 65535]");
+  const int h = (int)(n / halves);
+  hipStream_t s = as_stream(stream);
+  if (dtype == HIPMC_F32)
+    return rhat_run(h, halves, (int)chains, (int)dims, stride_n, stride_chain,
+                    stride_dim, (const float*)x, chunks, ws_sums, out, s);
+  return rhat_run(h, halves, (int)chains, (int)dims, stride_n, stride_chain,
+                  stride_dim, (const double*)x, chunks, ws_sums, out, s);
+}
+
+}  // extern "C"

@@ -4,13 +4,16 @@
 Same formulas as the reference: centred FFT auto-covariance zero-padded to
 2^ceil(log2(2n)) divided by (n - k); cross-chain ESS (Vehtari et al. 2021
 eq. 10) truncated at the first negative auto-correlation; split R-hat.
-Computed in float64 on the GPU with torch.fft (these run once per sampling
-run, on the traced draws).
+Computed in float64: float32 and float64 draws on the GPU by libhipmc
+(csrc/diagnostic.hip: the cross-chain ESS of up to 4096 draws, and R-hat),
+everything else with torch.
 """
 
 import math
 
 import torch
+
+from probability_amd import _lib
 
 __all__ = ['effective_sample_size', 'potential_scale_reduction']
 
@@ -19,6 +22,73 @@ def _as64(x):
   if isinstance(x, torch.Tensor):
     return x.to(torch.float64)
   return torch.as_tensor(x, dtype=torch.float64)
+
+
+# The most draws whose zero-padded transform fits in one workgroup's LDS.
+_MAX_DRAWS = 4096
+
+
+def _on_device(x):
+  """Whether the kernels take x: a plain float tensor on the GPU that no
+  transformation (autograd, forward mode, vmap, tracing) follows."""
+  return (type(x) is torch.Tensor and x.is_cuda and
+          x.dtype in (torch.float32, torch.float64) and
+          not (x.requires_grad and torch.is_grad_enabled()) and
+          torch.autograd.forward_ad._current_level < 0 and
+          not torch._C._functorch.is_functorch_wrapped_tensor(x) and
+          not torch.compiler.is_compiling())
+
+
+def _series(x, chain_axes):
+  """x [n, chain axes..., rest...] as [n, chains, dims] (a view where the
+  strides allow)."""
+  chains = math.prod(x.shape[1:1 + chain_axes])
+  return x.reshape(x.shape[0], chains, math.prod(x.shape[1 + chain_axes:]))
+
+
+def _ess_device(states, filter_threshold):
+  """states [n, chains, ...] -> cross-chain ESS [...]."""
+  x = _series(states, 1)
+  n, c, d = x.shape
+  # blocks that share a dimension's pairs of chains: two blocks a CU are
+  # resident, so up to 512 run at once; none is empty
+  pairs = (c + 1) // 2
+  per = -(-pairs // min(pairs, max(1, 512 // d)))
+  blocks = -(-pairs // per)
+  m = max(16, 1 << (2 * n - 1).bit_length())
+  f64 = dict(dtype=torch.float64, device=x.device)
+  rows = torch.empty((d, c, n), dtype=x.dtype, device=x.device)
+  means = torch.empty((d, c), **f64)
+  power = torch.empty((blocks, d, m), **f64)
+  out = torch.empty(d, **f64)
+  with torch.cuda.device(x.device):
+    _lib.check(_lib.lib().hipmc_effective_sample_size(
+        _lib.dtype_code(x.dtype), n, c, d, *x.stride(), _lib.ptr(x),
+        0 if filter_threshold is None else 1,
+        0.0 if filter_threshold is None else float(filter_threshold), blocks,
+        _lib.ptr(rows), _lib.ptr(means), _lib.ptr(power), _lib.ptr(out),
+        _lib.stream_handle(x.device)))
+  return out.reshape(states.shape[2:])
+
+
+def _rhat_device(state, independent_chain_ndims, split_chains):
+  """state [n, chain axes..., ...] -> R-hat [...]."""
+  x = _series(state, independent_chain_ndims)
+  n, c, d = x.shape
+  halves = 2 if split_chains else 1
+  # time chunks so that about 2048 blocks of 64 series run, each with at
+  # least 32 draws
+  blocks = halves * (-(-(c * d) // 64))
+  chunks = max(1, min(2048 // blocks, (n // halves) // 32))
+  sums = torch.empty((chunks, halves, 2, c * d), dtype=torch.float64,
+                     device=x.device)
+  out = torch.empty(d, dtype=torch.float64, device=x.device)
+  with torch.cuda.device(x.device):
+    _lib.check(_lib.lib().hipmc_potential_scale_reduction(
+        _lib.dtype_code(x.dtype), n, c, d, *x.stride(), _lib.ptr(x),
+        1 if split_chains else 0, chunks, _lib.ptr(sums), _lib.ptr(out),
+        _lib.stream_handle(x.device)))
+  return out.reshape(state.shape[1 + independent_chain_ndims:])
 
 
 def auto_covariance(x):
@@ -47,6 +117,10 @@ def _flatten_chain_dims(states, cross_chain_dims):
 
 
 def _ess_one(states, cross_chain_dims, filter_threshold):
+  if cross_chain_dims is not None and _on_device(states) and states.dim() > 1:
+    x = _flatten_chain_dims(states, cross_chain_dims)
+    if 1 <= x.shape[0] <= _MAX_DRAWS and x.shape[1] >= 2 and x.numel() > 0:
+      return _ess_device(x, filter_threshold)
   states = _as64(states)
   if cross_chain_dims is not None:
     states = _flatten_chain_dims(states, cross_chain_dims)
@@ -89,7 +163,7 @@ def effective_sample_size(states, filter_threshold=0., filter_beyond_lag=None,
 
 
 def _rhat_one(state, independent_chain_ndims, split_chains):
-  x = _as64(state)
+  x = state if _on_device(state) else _as64(state)
   icn = independent_chain_ndims
   if icn < 1:
     raise ValueError('Argument `independent_chain_ndims` must be `>= 1`, '
@@ -102,6 +176,12 @@ def _rhat_one(state, independent_chain_ndims, split_chains):
     if n < 4:
       raise ValueError('Must provide at least 4 samples when splitting '
                        'chains. Found {}'.format(n))
+  if _on_device(x):
+    if x.numel() > 0 and isinstance(icn, int) and icn < x.dim():
+      return _rhat_device(x, icn, split_chains)
+    x = _as64(x)
+  if split_chains:
+    n = x.shape[0]
     x = x[:n - n % 2]
     x = x.reshape((2, n // 2) + tuple(x.shape[1:])).transpose(0, 1)
     icn += 1
