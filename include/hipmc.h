@@ -504,6 +504,59 @@ int hipmc_draws(int32_t dtype, int32_t kind, const uint32_t seed[2],
                 int32_t index, void* out, uint8_t* out_aux, uint64_t stream);
 
 /*
+ * Tiled evaluation of many chains of a regression (LOGISTIC / LINEAR): the
+ * logits and the gradients as matrix products over tiles of 16 or 32 chains
+ * and ranges of rows, in the state's precision.  dim_x <= 256 (F32) / 128
+ * (F64).  Results equal hipmc_target_eval / hipmc_hmc_run /
+ * hipmc_leapfrog_run up to the order of floating-point sums.
+ * hipmc_glm_tile_plan gives the tiles, row ranges and workspace of a launch
+ * of n_chains chains of one problem (they depend on its arguments only);
+ * n_obs and dim_x are the table's, which is in device memory.
+ */
+typedef struct hipmc_glm_plan {
+  int32_t tile_chains;
+  int32_t width;          /* columns of a partial gradient row */
+  int32_t n_tiles;
+  int32_t n_split;        /* row ranges */
+  int32_t rows_per_split;
+  int32_t pad_;
+  int64_t workspace_bytes;
+} hipmc_glm_plan;
+
+int hipmc_glm_tile_plan(int32_t dtype, int32_t n_obs, int32_t dim_x,
+                        int32_t n_chains, int32_t dim_stride,
+                        int32_t trajectory, hipmc_glm_plan* plan);
+
+/* Log density and gradient at x [n_chains, dim_stride] of problems[0]. */
+int hipmc_glm_tile_eval(int32_t dtype, const hipmc_problem* problems,
+                        int32_t n_obs, int32_t dim_x, int32_t dim,
+                        int32_t n_chains, int32_t dim_stride, const void* x,
+                        void* out_tlp, void* out_grad, void* ws,
+                        int64_t ws_bytes, uint64_t stream);
+
+/* The same for a batch of problems: tiles (device, int32 [n_tiles, 8]) rows
+ * {problem, first chain, chains (1..tile_chains), row ranges
+ * (1..max_split), first slot, rows per range (a multiple of 64), 0, 0}; a
+ * tile's ranges take consecutive slots below n_slots.  ws_grad: dtype
+ * [n_slots, tile_chains, width]; ws_sum: float64 [n_slots, tile_chains];
+ * width: a multiple of 16 that holds every problem's coefficients, at most
+ * 128 (F32) / 64 (F64) with tiles of 32 chains. */
+int hipmc_glm_tile_eval_batch(int32_t dtype, const hipmc_problem* problems,
+                              const int32_t* tiles, int32_t n_tiles,
+                              int32_t max_split, int32_t n_slots,
+                              int32_t tile_chains, int32_t width,
+                              int32_t max_dim, int32_t dim_stride,
+                              const void* x, void* out_tlp, void* out_grad,
+                              void* ws_grad, double* ws_sum, uint64_t stream);
+
+/* hipmc_hmc_run (calibrated != 0) or hipmc_leapfrog_run over one problem (no
+ * chain maps or streams) with at least one leapfrog step: one gradient launch
+ * for all chains and one per-chain launch per leapfrog step. */
+int hipmc_glm_tile_hmc_run(const hipmc_run_args* args, int32_t calibrated,
+                           int32_t n_obs, int32_t dim_x, void* ws,
+                           int64_t ws_bytes, uint64_t stream);
+
+/*
  * Cross-chain effective sample size of draws x (dtype; element (t, c, d) at
  * t * stride_n + c * stride_chain + d * stride_dim, strides in elements), all
  * in float64: per dimension d the autocovariance averaged over the chains, its

@@ -32,7 +32,9 @@ EXPORTED_SYMBOLS = (
     'hipmc_da_update', 'hipmc_simple_step_update', 'hipmc_mh_accept',
     'hipmc_bijector', 'hipmc_draws', 'hipmc_moments_update',
     'hipmc_variance_update', 'hipmc_glm_hmc_run_noalloc',
-    'hipmc_effective_sample_size', 'hipmc_potential_scale_reduction')
+    'hipmc_effective_sample_size', 'hipmc_potential_scale_reduction',
+    'hipmc_glm_tile_plan', 'hipmc_glm_tile_eval',
+    'hipmc_glm_tile_eval_batch', 'hipmc_glm_tile_hmc_run')
 
 _vp = ctypes.c_void_p
 _i32 = ctypes.c_int32
@@ -104,6 +106,14 @@ class GlmHmcArgs(ctypes.Structure):
   ]
 
 
+class GlmPlan(ctypes.Structure):
+  _fields_ = [
+      ('tile_chains', _i32), ('width', _i32), ('n_tiles', _i32),
+      ('n_split', _i32), ('rows_per_split', _i32), ('pad_', _i32),
+      ('workspace_bytes', _i64),
+  ]
+
+
 class HipmcError(RuntimeError):
   pass
 
@@ -150,6 +160,15 @@ def lib():
       l.hipmc_potential_scale_reduction.argtypes = [
           _i32, _i64, _i64, _i64, _i64, _i64, _i64, _vp, _i32, _i32, _vp, _vp,
           _u64]
+      l.hipmc_glm_tile_plan.argtypes = [_i32, _i32, _i32, _i32, _i32, _i32,
+                                        ctypes.POINTER(GlmPlan)]
+      l.hipmc_glm_tile_eval.argtypes = [_i32, _vp, _i32, _i32, _i32, _i32,
+                                        _i32, _vp, _vp, _vp, _vp, _i64, _u64]
+      l.hipmc_glm_tile_eval_batch.argtypes = [
+          _i32, _vp, _vp, _i32, _i32, _i32, _i32, _i32, _i32, _i32, _vp, _vp,
+          _vp, _vp, _vp, _u64]
+      l.hipmc_glm_tile_hmc_run.argtypes = [ctypes.POINTER(RunArgs), _i32, _i32,
+                                           _i32, _vp, _i64, _u64]
       l.hipmc_bijector.argtypes = [_i32, _vp, _vp, _i32, _i32, _i32, _i32,
                                    _vp, _vp, _u64]
       l.hipmc_draws.argtypes = [_i32, _i32, _vp, _i32, _i32, _i32, _i32, _i32,

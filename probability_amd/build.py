@@ -2,7 +2,8 @@
 
 The library is linked from several objects compiled in parallel: the ABI
 and small kernels (hipmc.hip), the BF16 MFMA path (mfma.hip), the
-convergence diagnostics (diagnostic.hip) and the sampling kernels, one object per (kernel group, dtype, target family) from
+convergence diagnostics (diagnostic.hip), the tiled GLM evaluation (one
+object per type from glm_tile.hip) and the sampling kernels, one object per (kernel group, dtype, target family) from
 inst.hip.
 
 Usage: python -m probability_amd.build   (or probability_amd.build.build()).
@@ -33,6 +34,9 @@ def objects():
   """(object name, source, extra defines) of every object of the library."""
   out = [('hipmc', 'hipmc.hip', []), ('mfma', 'mfma.hip', []),
          ('diagnostic', 'diagnostic.hip', [])]
+  for t in ('float', 'double'):
+    out.append((f'glm_tile_{t[0]}{"32" if t == "float" else "64"}',
+                'glm_tile.hip', [f'-DHIPMC_INST_T={t}']))
   for group, nuts in (('nuts', 1), ('hmc', 0)):
     for t in ('float', 'double'):
       for fam, code in _FAMILIES.items():

@@ -133,6 +133,80 @@ struct EvalL {
   }
 };
 
+// ------------------------------------------------------ tiled GLM evaluation
+size_t round256(size_t n) { return (n + 255) & ~(size_t)255; }
+
+// Tiles and row ranges of a launch of n_chains chains of one problem, and the
+// workspace: partial gradients, partial sums, and for trajectories the
+// positions, momenta and initial kinetic energies.
+// * 32 chains a tile where two groups' coefficients and gradients fit a wave's
+//   registers (8 slabs of 16 float32, 4 of float64), else 16.
+// * Row ranges so that about 512 blocks run (two a CU) where that leaves each
+//   at least eight passes of its waves, else 256, none shorter than one pass:
+//   a block's fixed part (coefficients in, partial sums out) costs about two
+//   passes.  Log density and gradient, us, 512 against 256 blocks: 2048 x 64,
+//   1024 chains 19.9 / 17.3; 6001 x 101, 512 chains 30.2 / 28.2; 8192 x 128,
+//   2048 chains 98.7 / 101.6; float64 8000 x 127, 1000 chains 131 / 146.
+// They depend on the problem's own sizes and chain count only.
+int plan_tiles(int32_t dtype, int32_t n_obs, int32_t dim_x, int32_t n_chains,
+               int32_t dim_stride, bool trajectory, hipmc_glm_plan* p) {
+  if (dtype != HIPMC_F32 && dtype != HIPMC_F64)
+    return fail(HIPMC_E_INVALID, "glm_tile: bad dtype");
+  if (n_obs < 1 || dim_x < 1 || n_chains < 1 || dim_stride < dim_x)
+    return fail(HIPMC_E_INVALID,
+                "glm_tile: need n_obs, dim_x, n_chains >= 1 and "
+                "dim_stride >= dim_x");
+  const bool f32 = dtype == HIPMC_F32;
+  const int slabs = (dim_x + 15) / 16;
+  if (slabs > (f32 ? 16 : 8))
+    return fail(HIPMC_E_UNSUPPORTED,
+                "glm_tile: too many coefficients for the tiled evaluation");
+  p->tile_chains = n_chains > 16 && slabs <= (f32 ? 8 : 4) ? 32 : 16;
+  p->width = 16 * slabs;
+  p->n_tiles = (n_chains + p->tile_chains - 1) / p->tile_chains;
+  const int most = (n_obs + kTileRows - 1) / kTileRows;
+  auto rows_of = [&](int blocks) {
+    int split = blocks / p->n_tiles;
+    split = split < 1 ? 1 : (split > most ? most : split);
+    const int rows = (n_obs + split - 1) / split;
+    return (rows + kTileRows - 1) / kTileRows * kTileRows;
+  };
+  p->rows_per_split = rows_of(512);
+  if (p->rows_per_split < 8 * kTileRows) p->rows_per_split = rows_of(256);
+  p->n_split = (n_obs + p->rows_per_split - 1) / p->rows_per_split;
+  const size_t es = f32 ? 4 : 8;
+  const size_t part = (size_t)p->n_tiles * p->n_split * p->tile_chains;
+  size_t bytes = round256(part * p->width * es) + round256(part * 8);
+  if (trajectory)
+    bytes += 2 * round256((size_t)n_chains * dim_stride * es) +
+             round256((size_t)n_chains * 8);
+  p->workspace_bytes = (int64_t)bytes;
+  return HIPMC_OK;
+}
+
+// The launch arguments of a plan over a workspace; returns its next free byte.
+unsigned char* tile_args(const hipmc_glm_plan& p, int32_t dtype,
+                         const hipmc_problem* problems, int32_t n_chains,
+                         int32_t dim_stride, const void* x, void* ws,
+                         GlmTileArgs* a) {
+  const size_t es = dtype == HIPMC_F32 ? 4 : 8;
+  const size_t part = (size_t)p.n_tiles * p.n_split * p.tile_chains;
+  unsigned char* w = (unsigned char*)ws;
+  a->problems = problems;
+  a->tiles = nullptr;
+  a->n_tiles = p.n_tiles;
+  a->n_split = p.n_split;
+  a->rows = p.rows_per_split;
+  a->n_chains = n_chains;
+  a->stride = dim_stride;
+  a->width = p.width;
+  a->x = x;
+  a->ws_grad = w;
+  w += round256(part * p.width * es);
+  a->ws_sum = (double*)w;
+  return w + round256(part * 8);
+}
+
 // ------------------------------------------------------------ DA kernel
 // reduce_logmeanexp of hmc_like_log_accept_prob_getter_fn(lar) over chains
 // [b, e) (`simple_step_size_adaptation.py:42-48`, `math/generic.py:221-273`),
@@ -650,6 +724,113 @@ int hipmc_target_eval(int32_t dtype, int32_t target_kind,
   return by_family<EvalL>(dtype, target_kind, k, problems, chain_problem,
                          n_chains, dim_stride, x, out_tlp, out_grad,
                          as_stream(stream));
+}
+
+int hipmc_glm_tile_plan(int32_t dtype, int32_t n_obs, int32_t dim_x,
+                        int32_t n_chains, int32_t dim_stride,
+                        int32_t trajectory, hipmc_glm_plan* plan) {
+  if (!plan) return fail(HIPMC_E_INVALID, "glm_tile: plan is NULL");
+  return plan_tiles(dtype, n_obs, dim_x, n_chains, dim_stride, trajectory != 0,
+                    plan);
+}
+
+int hipmc_glm_tile_eval(int32_t dtype, const hipmc_problem* problems,
+                        int32_t n_obs, int32_t dim_x, int32_t dim,
+                        int32_t n_chains, int32_t dim_stride, const void* x,
+                        void* out_tlp, void* out_grad, void* ws,
+                        int64_t ws_bytes, uint64_t stream) {
+  hipmc_glm_plan p;
+  const int rc = plan_tiles(dtype, n_obs, dim_x, n_chains, dim_stride, false,
+                            &p);
+  if (rc != HIPMC_OK) return rc;
+  if (!problems || !x || !ws)
+    return fail(HIPMC_E_INVALID, "glm_tile: NULL argument");
+  if (dim < dim_x || dim > dim_stride)
+    return fail(HIPMC_E_INVALID, "glm_tile: need dim_x <= dim <= dim_stride");
+  if (ws_bytes < p.workspace_bytes)
+    return fail(HIPMC_E_INVALID, "glm_tile: workspace too small");
+  GlmTileArgs a;
+  tile_args(p, dtype, problems, n_chains, dim_stride, x, ws, &a);
+  const int k = pick_k(dim, kFamilyGlm);
+  hipStream_t s = as_stream(stream);
+  return dtype == HIPMC_F32
+             ? glm_tile_eval<float>(a, p.tile_chains, k, out_tlp, out_grad, s)
+             : glm_tile_eval<double>(a, p.tile_chains, k, out_tlp, out_grad, s);
+}
+
+int hipmc_glm_tile_eval_batch(int32_t dtype, const hipmc_problem* problems,
+                              const int32_t* tiles, int32_t n_tiles,
+                              int32_t max_split, int32_t n_slots,
+                              int32_t tile_chains, int32_t width,
+                              int32_t max_dim, int32_t dim_stride,
+                              const void* x, void* out_tlp, void* out_grad,
+                              void* ws_grad, double* ws_sum, uint64_t stream) {
+  if (dtype != HIPMC_F32 && dtype != HIPMC_F64)
+    return fail(HIPMC_E_INVALID, "glm_tile: bad dtype");
+  if (!problems || !tiles || !x || !ws_grad || !ws_sum)
+    return fail(HIPMC_E_INVALID, "glm_tile: NULL argument");
+  if (n_tiles < 1 || max_split < 1 || n_slots < n_tiles || max_dim < 1 ||
+      max_dim > dim_stride || width < 16 || width % 16 ||
+      (tile_chains != 16 && tile_chains != 32) ||
+      (int64_t)n_tiles * max_split > 0x7fffffff)
+    return fail(HIPMC_E_INVALID, "glm_tile: bad tile table");
+  const int k = pick_k(max_dim, kFamilyGlm);
+  if (k < 0) return fail(HIPMC_E_UNSUPPORTED, "glm_tile: state too wide");
+  GlmTileArgs a;
+  a.problems = problems;
+  a.tiles = (const GlmTile*)tiles;
+  a.n_tiles = n_tiles;
+  a.n_split = max_split;
+  a.rows = 0;
+  a.n_chains = 0;
+  a.stride = dim_stride;
+  a.width = width;
+  a.x = x;
+  a.ws_grad = ws_grad;
+  a.ws_sum = ws_sum;
+  hipStream_t s = as_stream(stream);
+  return dtype == HIPMC_F32
+             ? glm_tile_eval<float>(a, tile_chains, k, out_tlp, out_grad, s)
+             : glm_tile_eval<double>(a, tile_chains, k, out_tlp, out_grad, s);
+}
+
+int hipmc_glm_tile_hmc_run(const hipmc_run_args* a, int32_t calibrated,
+                           int32_t n_obs, int32_t dim_x, void* ws,
+                           int64_t ws_bytes, uint64_t stream) {
+  int rc = check_run(a, false);
+  if (rc) return rc;
+  if (a->target_kind != HIPMC_TARGET_LOGISTIC &&
+      a->target_kind != HIPMC_TARGET_LINEAR)
+    return fail(HIPMC_E_INVALID, "glm_tile: not a regression");
+  if (a->n_problems != 1 || a->chain_problem || a->chain_local || a->streams ||
+      a->chain_row || a->num_leapfrog_steps < 1)
+    return fail(HIPMC_E_INVALID,
+                "glm_tile: one problem, no chain maps or streams, at least "
+                "one leapfrog step");
+  if (!calibrated && a->n_iters != 1)
+    return fail(HIPMC_E_INVALID, "glm_tile: a proposal takes n_iters 1");
+  if (a->n_chains == 0) return HIPMC_OK;
+  hipmc_glm_plan p;
+  rc = plan_tiles(a->dtype, n_obs, dim_x, a->n_chains, a->dim_stride, true,
+                  &p);
+  if (rc != HIPMC_OK) return rc;
+  if (!ws || ws_bytes < p.workspace_bytes)
+    return fail(HIPMC_E_INVALID, "glm_tile: workspace too small");
+  const size_t rows_bytes = round256((size_t)a->n_chains * a->dim_stride *
+                                     (a->dtype == HIPMC_F32 ? 4 : 8));
+  GlmTileArgs t;
+  unsigned char* w = tile_args(p, a->dtype, a->problems, a->n_chains,
+                               a->dim_stride, nullptr, ws, &t);
+  t.x = w;
+  void* ws_p = w + rows_bytes;
+  double* ws_ke0 = (double*)(w + 2 * rows_bytes);
+  const int k = pick_k(a->max_dim, kFamilyGlm);
+  hipStream_t s = as_stream(stream);
+  return a->dtype == HIPMC_F32
+             ? glm_tile_hmc<float>(*a, t, p.tile_chains, k, calibrated != 0,
+                                   ws_p, ws_ke0, s)
+             : glm_tile_hmc<double>(*a, t, p.tile_chains, k, calibrated != 0,
+                                    ws_p, ws_ke0, s);
 }
 
 int hipmc_da_update(int32_t dtype, int32_t n_groups, const int32_t* step_group,

@@ -49,6 +49,40 @@ int launch_eval_k(int k, const hipmc_problem* p, const int32_t* cp, int n,
                   int stride, const void* x, void* tlp, void* grad,
                   hipStream_t s);
 
+// The tiled GLM evaluation (glm_tile.h): blocks of kTileWaves waves.
+constexpr int kTileWaves = 4;
+// Rows of a block's pass over its range: 16 per wave.
+constexpr int kTileRows = 16 * kTileWaves;
+
+// One tile of chains of a batch (device table, [n_tiles]); a launch over one
+// problem has none and works its tiles out.
+struct GlmTile {
+  int32_t prob, chain0, n_chains, n_split, slot0, rows, pad0_, pad1_;
+};
+static_assert(sizeof(GlmTile) == 32, "GlmTile layout");
+
+struct GlmTileArgs {
+  const hipmc_problem* problems;
+  const GlmTile* tiles;  // NULL: tiles of problem 0
+  int n_tiles, n_split;  // n_split: of every tile (NULL table) or the most
+  int rows;              // rows per split (NULL table)
+  int n_chains, stride;  // positions x [n_chains, stride]
+  int width;             // workspace row of a chain (16 * slabs)
+  const void* x;
+  void* ws_grad;    // T [slots, tile chains, width]
+  double* ws_sum;   // [slots, tile chains]
+};
+
+// Log density and gradient of every chain of the tiles; trajectories of a
+// run over one problem (glm_tile.hip).  ct: chains per tile (16 or 32); k:
+// register slots of the per-chain kernels.
+template <typename T>
+int glm_tile_eval(const GlmTileArgs& a, int ct, int k, void* tlp,
+                  void* grad_out, hipStream_t s);
+template <typename T>
+int glm_tile_hmc(const hipmc_run_args& r, const GlmTileArgs& a, int ct, int k,
+                 bool calibrated, void* ws_p, double* ws_ke0, hipStream_t s);
+
 // The BF16 MFMA logistic-regression HMC path (mfma.hip), with caller
 // workspaces or with the library's static scratch.
 int launch_glm_hmc(const hipmc_glm_hmc_args* a, hipStream_t s);

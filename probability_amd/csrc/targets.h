@@ -152,11 +152,23 @@ struct GroupLayout {
   }
 };
 
+// Sums over the rows of X that glm_tile_grad has left for a GLM evaluation
+// (G = kRowSums): this lane's elements of X^T (y - mean), and the
+// log-likelihood (logistic) or residual sum of squares (linear).
+constexpr int kRowSums = 0;
+template <typename T, int K, int G>
+struct RowSums {};
+template <typename T, int K>
+struct RowSums<T, K, kRowSums> {
+  T row_grad[K];
+  double row_sum;
+};
+
 // G > 1: the GLM target of a chain group (nuts_group_kernel); every
 // evaluation is a round in which all waves of the block pass over X for all
-// G chains.
+// G chains.  G = kRowSums: the sums over the rows are given.
 template <typename T, int K, int FAM, int G = 1>
-struct Target {
+struct Target : RowSums<T, K, G> {
   int kind, dim, n_obs;
   T p0, p1;
   double log_norm;
@@ -787,6 +799,9 @@ struct Target {
   // added in a fixed order.
   template <bool LINEAR>
   __device__ double glm(const T (&th)[K], T (&g)[K], double& lpu) {
+    if constexpr (G == kRowSums) {
+      return glm_given<LINEAR>(th, g, lpu);
+    }
     if constexpr (G > 1) {
       return glm_grouped<LINEAR>(th, g, lpu);
     }
@@ -918,6 +933,50 @@ struct Target {
       lp += -(double)n * (double)log(sigma) +
             (double)(T(-0.5) * (sigma / ss) * (sigma / ss));
       if (sigma < T(0)) lp = neg_inf();
+    }
+    lpu = lp;
+    return lpl;
+  }
+
+  // The terms of glm() around given sums over the rows.
+  template <bool LINEAR>
+  __device__ double glm_given(const T (&th)[K], T (&g)[K], double& lpu) {
+    const int lane = lane_id();
+    const int dx = LINEAR ? dim - 1 : dim;
+    T sigma = T(1), inv_s2 = T(1);
+    if (LINEAR) {
+#pragma unroll
+      for (int k = 0; k < K; ++k)
+        if (k == (dx >> 6)) sigma = readlane(th[k], dx & 63);
+      inv_s2 = T(1) / (sigma * sigma);
+    }
+    double lpl = 0.0;
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      const int e = k * 64 + lane;
+      const bool isb = e < dx;
+      const T bv = th[k] * inv_s0;
+      const T gl = LINEAR ? this->row_grad[k] * inv_s2 : this->row_grad[k];
+      lpl += isb ? (double)(T(-0.5) * bv * bv) : 0.0;
+      g[k] = isb ? gl - th[k] * inv_s0sq : T(0);
+    }
+    double lp = log_norm;
+    if (LINEAR) {
+      // the residual sum is float64, and so is the small difference of
+      // large terms that is its gradient
+      const double sd = (double)sigma;
+      const T ss = p1;
+      const T gs = (T)(this->row_sum / (sd * sd * sd) - (double)n_obs / sd -
+                       sd / ((double)ss * (double)ss));
+#pragma unroll
+      for (int k = 0; k < K; ++k)
+        if (k == (dx >> 6) && lane == (dx & 63)) g[k] = gs;
+      lp += -0.5 * this->row_sum / (sd * sd) -
+            (double)n_obs * (double)log(sigma) +
+            (double)(T(-0.5) * (sigma / ss) * (sigma / ss));
+      if (sigma < T(0)) lp = neg_inf();
+    } else {
+      lp += this->row_sum;
     }
     lpu = lp;
     return lpl;

@@ -8,6 +8,7 @@ import numpy as np
 import torch
 
 from probability_amd import _lib
+from probability_amd import glm_tile
 from probability_amd import tuning
 
 _OUT_FIELDS = ('out_log_accept_ratio', 'out_leapfrogs', 'out_is_accepted',
@@ -78,6 +79,17 @@ class Run:
     self.outputs[name] = t
     setattr(self.args, name, t.data_ptr())
     return t
+
+  def call_hmc(self, calibrated):
+    """hipmc_hmc_run or hipmc_leapfrog_run, or the tiled trajectories where
+    those are faster."""
+    a = self.args
+    if glm_tile.takes_trajectory(self.spec, a.max_dim, self.n_chains,
+                                 a.num_leapfrog_steps):
+      glm_tile.run_hmc(self.spec, a, calibrated, self.state.device)
+      return self.outputs
+    return self.call(_lib.lib().hipmc_hmc_run if calibrated
+                     else _lib.lib().hipmc_leapfrog_run)
 
   def call(self, fn):
     _lib.check(fn(self.args, _lib.stream_handle(self.state.device)))

@@ -22,6 +22,7 @@ import torch
 from probability_amd import _lib
 from probability_amd import tuning
 from probability_amd import bijectors as bij_lib
+from probability_amd import glm_tile
 from probability_amd import random as samplers
 from probability_amd import targets as targets_lib
 
@@ -111,6 +112,13 @@ class PosteriorBatch:
     self.kind = self.specs[0].kind
     if _family(self.kind) == 2 and len({s.kind for s in self.specs}) > 1:
       self.kind = _lib.TARGET_DIAG_NORMAL
+    self._tiles = None  # of eval()
+    if fams == {1}:
+      cols = max(d - (s.kind == _lib.TARGET_LINEAR)
+                 for s, d in zip(self.specs, self.dims))
+      self._tiles = glm_tile.BatchTiles([s.base.n_obs for s in self.specs],
+                                        cols, self.num_chains, offs,
+                                        self.dtype, self.device)
     g = int(chains_per_block or 1)
     if g not in (1, 2, 4):
       raise ValueError('chains_per_block must be 1, 2 or 4')
@@ -134,6 +142,16 @@ class PosteriorBatch:
 
   def eval(self, x):
     """(tlp [C], grad [C, dim_stride]) of every chain at x."""
+    if self._tiles is None or self._tiles.table is None:
+      return self.eval_chains(x)
+    tlp = torch.empty(self.n_chains, dtype=self.dtype, device=self.device)
+    grad = torch.zeros_like(x)
+    self._tiles.evaluate(self, x, tlp, grad)
+    return tlp, grad
+
+  def eval_chains(self, x):
+    """eval by the samplers' own per-chain pass, whose sums do not depend on
+    the batch (a run starts from them, so that its draws do not either)."""
     tlp = torch.empty(self.n_chains, dtype=self.dtype, device=self.device)
     grad = torch.zeros_like(x)
     _lib.check(_lib.lib().hipmc_target_eval(
@@ -289,7 +307,7 @@ class RaggedRun:
       for _, _, r in self.runs:
         with torch.cuda.stream(r.stream):
           r.x.copy_(_init_uniform(r.batch, setup_seed))
-          r.tlp, r.grad = r.batch.eval(r.x)
+          r.tlp, r.grad = r.batch.eval_chains(r.x)
 
   @property
   def t(self):
@@ -469,7 +487,7 @@ class _Run:
       else:
         self.x = batch.bijector(torch.as_tensor(init_state, dtype=dt,
                                                 device=dev).contiguous(), 1)
-      self.tlp, self.grad = batch.eval(self.x)
+      self.tlp, self.grad = batch.eval_chains(self.x)
       self.step = torch.as_tensor(np.broadcast_to(
           np.asarray(step_size, np.float64), (p,)).copy(),
                                   device=dev).to(dt)

@@ -14,7 +14,6 @@ import collections
 
 import torch
 
-from probability_amd import _lib
 from probability_amd import random as samplers
 from probability_amd import targets as targets_lib
 from probability_amd.mcmc import kernel as kernel_base
@@ -104,7 +103,7 @@ class UncalibratedHamiltonianMonteCarlo(kernel_base.TransitionKernel):
     corr = run.want('out_energy', (1, c), spec.dtype)
     p0 = run.want('out_initial_momentum', (c, d), spec.dtype)
     p1 = run.want('out_final_momentum', (c, d), spec.dtype)
-    run.call(_lib.lib().hipmc_leapfrog_run)
+    run.call_hmc(False)
     chain_shape = tuple(previous_kernel_results.target_log_prob.shape)
     next_parts = spec.unpack_state(state, chain_shape)
     results = previous_kernel_results._replace(
@@ -210,7 +209,7 @@ class HamiltonianMonteCarlo(kernel_base.TransitionKernel):
     ptlp = run.want('out_proposed_tlp', (c,), spec.dtype)
     p0 = run.want('out_initial_momentum', (c, d), spec.dtype)
     p1 = run.want('out_final_momentum', (c, d), spec.dtype)
-    run.call(_lib.lib().hipmc_hmc_run)
+    run.call_hmc(True)
     cs = tuple(acc.target_log_prob.shape)
     accepted = is_acc.reshape(cs).bool()
     proposed_results = acc._replace(

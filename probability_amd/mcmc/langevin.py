@@ -17,7 +17,6 @@ import math
 
 import torch
 
-from probability_amd import _lib
 from probability_amd import random as samplers
 from probability_amd import targets as targets_lib
 from probability_amd.mcmc import _runner
@@ -111,7 +110,7 @@ class UncalibratedLangevin(kernel_base.TransitionKernel):
     run.args.num_leapfrog_steps = 1
     c, _ = state.shape
     corr = run.want('out_energy', (1, c), spec.dtype)
-    run.call(_lib.lib().hipmc_leapfrog_run)
+    run.call_hmc(False)
     cs = tuple(pkr.target_log_prob.shape)
     if not self.compute_acceptance:
       corr = torch.zeros_like(corr)
@@ -179,7 +178,7 @@ class MetropolisAdjustedLangevinAlgorithm(kernel_base.TransitionKernel):
     corr = run.want('out_energy', (1, c), spec.dtype)
     pst = run.want('out_proposed_state', (c, d), spec.dtype)
     ptlp = run.want('out_proposed_tlp', (c,), spec.dtype)
-    run.call(_lib.lib().hipmc_hmc_run)
+    run.call_hmc(True)
     cs = tuple(acc.target_log_prob.shape)
     accepted = is_acc.reshape(cs).bool()
     # the proposal's gradient is not kept by the fused launch (the accepted

@@ -292,8 +292,6 @@ def _run_fused(plan, num_results, current_state, num_burnin_steps, thin,
   else:
     n_adapt = 0
 
-  fn = (_lib.lib().hipmc_nuts_run if plan.kind == 'nuts'
-        else _lib.lib().hipmc_hmc_run)
   # Large-batch logistic HMC runs its all-chain gradients as MFMA GEMMs.
   mfma = (plan.kind == 'hmc' and plan.ttk is None and
           isinstance(spec, targets_lib.LogisticRegressionBF16) and
@@ -327,7 +325,7 @@ def _run_fused(plan, num_results, current_state, num_burnin_steps, thin,
     else:
       _launch_fused(plan, spec, table, state, tlp, grad, step, base_seed, n,
                     t, lar_all, outs, trace_state, num_burnin_steps, thin,
-                    num_results, fn, stream, events)
+                    num_results, events)
     if plan.da is not None:
       _lib.check(_lib.lib().hipmc_da_update(
           _lib.dtype_code(dt), gplan.n_steps, _lib.ptr(gplan.step_group),
@@ -404,7 +402,7 @@ def _run_fused(plan, num_results, current_state, num_burnin_steps, thin,
 
 def _launch_fused(plan, spec, table, state, tlp, grad, step, base_seed, n, t,
                   lar_all, outs, trace_state, num_burnin_steps, thin,
-                  num_results, fn, stream, events):
+                  num_results, events):
   """One sampler launch of the fused loop over iterations [t, t + n)."""
   run = _runner.Run(spec, table, state, tlp, grad, step, base_seed,
                     n_iters=n, fold_seed=True, iter0=t,
@@ -426,7 +424,10 @@ def _launch_fused(plan, spec, table, state, tlp, grad, step, base_seed, n, t,
     e0 = torch.cuda.Event(enable_timing=True)
     e1 = torch.cuda.Event(enable_timing=True)
     e0.record()
-  _lib.check(fn(a, stream))
+  if plan.kind == 'nuts':
+    run.call(_lib.lib().hipmc_nuts_run)
+  else:
+    run.call_hmc(True)
   if events is not None:
     e1.record()
     events.append((e0, e1, t, n))

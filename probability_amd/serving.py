@@ -309,7 +309,7 @@ class SamplerServer:
       req.problem_bytes = bytes(tspec.problem(tspec.bijectors_for_eval()))
       x = torch.zeros((req.num_chains, req.spec.dim), dtype=self.dtype,
                       device=self.device)
-      tlp, grad = tspec.log_prob_and_grad_flat(x)
+      tlp, grad = tspec.log_prob_and_grad_chains(x)
       rows = torch.as_tensor(req.rows, device=self.device)
       pool.state[rows] = torch.nn.functional.pad(
           x, (0, pool.dim_stride - x.shape[1]))

@@ -20,6 +20,7 @@ import torch
 
 from probability_amd import _lib
 from probability_amd import bijectors as bij_lib
+from probability_amd import glm_tile
 
 _HALF_LOG_2PI = 0.5 * math.log(2.0 * math.pi)
 
@@ -123,14 +124,28 @@ class TargetSpec:
 
   def log_prob_and_grad_flat(self, x, bijectors=None):
     """x [C, dim] -> (tlp [C], grad [C, dim]) on the device."""
-    _lib.require_cuda()
+    return self._eval_flat(x, bijectors, True)
+
+  def log_prob_and_grad_chains(self, x, bijectors=None):
+    """log_prob_and_grad_flat by the samplers' own per-chain pass, whose sums
+    do not depend on how many chains are evaluated together: what starts a
+    run whose draws equal those of the same problem in any batch."""
+    return self._eval_flat(x, bijectors, False)
+
+  def _eval_flat(self, x, bijectors, tiled):
+    if not x.is_cuda:  # a tensor on the GPU shows that there is one
+      _lib.require_cuda()
     x = x.to(device=self.device, dtype=self.dtype).contiguous()
     c = x.shape[0]
     tlp = torch.empty(c, dtype=self.dtype, device=self.device)
     grad = torch.empty_like(x)
+    dim = self.dim
+    if (tiled and x.shape[1] >= dim and glm_tile.takes_eval(self, dim, c)):
+      glm_tile.evaluate(self, self.table(bijectors), x, tlp, grad)
+      return tlp, grad
     _lib.check(_lib.lib().hipmc_target_eval(
         _lib.dtype_code(self.dtype), self.kind,
-        _lib.ptr(self.table(bijectors)), None, c, x.shape[1], self.dim,
+        _lib.ptr(self.table(bijectors)), None, c, x.shape[1], dim,
         _lib.ptr(x), _lib.ptr(tlp), _lib.ptr(grad),
         _lib.stream_handle(self.device)))
     return tlp, grad
@@ -187,6 +202,10 @@ class TransformedTarget(TargetSpec):
 
   def log_prob_and_grad_flat(self, x, bijectors=None):
     return self._base.log_prob_and_grad_flat(
+        x, bijectors if bijectors is not None else self._bijectors)
+
+  def log_prob_and_grad_chains(self, x, bijectors=None):
+    return self._base.log_prob_and_grad_chains(
         x, bijectors if bijectors is not None else self._bijectors)
 
 
@@ -308,12 +327,12 @@ class LogisticRegressionBF16(LogisticRegression):
     return (self.dim == self.mfma_dim and n_chains % 64 == 0 and
             self.n_obs % 32 == 0 and self.dtype == torch.float32)
 
-  def log_prob_and_grad_flat(self, x, bijectors=None):
+  def _eval_flat(self, x, bijectors, tiled):
     if bijectors is None and self.mfma_ok(int(x.shape[0])):
       from probability_amd.mcmc import glm_mfma
       x = x.to(device=self.device, dtype=torch.float32).contiguous()
       return glm_mfma.GlmHmcRunner(self, x.shape[0]).bootstrap(x)
-    return super().log_prob_and_grad_flat(x, bijectors)
+    return super()._eval_flat(x, bijectors, tiled)
 
 
 class LinearRegression(_GlmData, TargetSpec):
