@@ -1,6 +1,6 @@
 // Large-batch HMC for Bayesian logistic regression with the design matrix
 // stored in BF16 and the all-chain contraction on MFMA (gfx950
-// v_mfma_f32_16x16x32_bf16).
+// v_mfma_f32_32x32x16_bf16).
 //
 // One leapfrog gradient for C chains (`mcmc/hmc.py` target gradient through
 // `mcmc/internal/util.py:246-308`, Bernoulli logits `bernoulli.py:119-135`):
@@ -16,6 +16,8 @@
 // data.
 #pragma once
 
+#include <type_traits>
+
 #include "../../include/hipmc.h"
 #include "common.h"
 
@@ -23,16 +25,40 @@ namespace hipmc {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 constexpr int kMD = 256;       // state dimension of this path
 constexpr int kMRows = 32;     // rows per LDS tile
-constexpr int kMChains = 64;   // chain granularity of the path (16 per wave)
+constexpr int kMChains = 64;   // chain granularity of the path (32 per wave)
 constexpr int kRPitch = kMRows + 8;    // bf16 per R row (one chain) in LDS
 
-__device__ inline f32x4 mfma16(const bf16x8& a, const bf16x8& b,
-                               const f32x4& c) {
-  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+// D += A B with A 32 x 16, B 16 x 32: lane l holds row l % 32 of A and column
+// l % 32 of B at k = 8 (l / 32) + [0, 8); register r of D is row
+// 8 (r / 4) + 4 (l / 32) + r % 4, column l % 32.
+// The unit adds its products to the accumulator in groups of 8 in the order
+// of k, so two of these in a row give bit for bit what one
+// v_mfma_f32_16x16x32_bf16 of the same 32 columns gives.
+__device__ inline f32x16 mfma32(const bf16x8& a, const bf16x8& b,
+                                const f32x16& c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
+}
+
+// Where element e of chain c stands in Bhi and Blo: in the order in which the
+// gradient's waves read their fragments, 32 chains by 16 elements per KiB.
+// (Read from rows, a load of 16 bytes per lane touched 32 cache lines, and a
+// launch with one tile per workgroup took 1 us longer.)
+__device__ inline size_t coef_index(int c, int e) {
+  return (size_t)(c >> 5) * 32 * kMD +
+         (((e >> 4) * 64 + ((e >> 3) & 1) * 32 + (c & 31)) * 8 + (e & 7));
+}
+
+// two floats rounded to BF16, the first in the low half
+__device__ inline uint32_t pack_bf16(float a, float b) {
+  const f32x2 v = {a, b};
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2));
 }
 
 // Direct global -> LDS loads (global_load_lds): the wave's 64 lanes each
@@ -46,6 +72,7 @@ __device__ inline f32x4 mfma16(const bf16x8& a, const bf16x8& b,
 // (no LDS-DMA builtins, no dynamically indexed register arrays), which the
 // gfx950 assembly of the kernel confirms (its only m0 writes are these).
 typedef __attribute__((address_space(3))) char lds_byte;
+typedef const __attribute__((address_space(3))) bf16x8 lds_bf16x8;
 __device__ inline uint32_t lds_addr(void* p) {
   return (uint32_t)(uintptr_t)(lds_byte*)p;
 }
@@ -53,200 +80,327 @@ __device__ inline void lds_dma16(const void* g, void* lds_base) {
   asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off"
                :: "v"(g), "s"(lds_addr(lds_base)) : "memory", "m0");
 }
-__device__ inline void lds_dma4(const void* g, void* lds_base) {
-  asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dword %0, off"
-               :: "v"(g), "s"(lds_addr(lds_base)) : "memory", "m0");
+// the same from a wave-uniform address plus 32-bit lane offsets
+__device__ inline void lds_dma16(const void* g, uint32_t off, void* lds_base) {
+  asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1"
+               :: "v"(off), "s"(g), "s"(lds_addr(lds_base))
+               : "memory", "m0");
+}
+__device__ inline void lds_dma4(const void* g, uint32_t off, void* lds_base) {
+  asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dword %0, %1"
+               :: "v"(off), "s"(g), "s"(lds_addr(lds_base))
+               : "memory", "m0");
 }
 
 // Chunk swizzle of X^T row d: 16 consecutive d of one chunk column land in
 // 16 distinct 16-byte bank groups, and any 8 consecutive aligned d in 8.
 __device__ inline int xt_swz(int d) { return ((d >> 1) ^ (d >> 2)) & 3; }
 
-// X tile: 16-byte chunk (row, c) at chunk row * 32 + (c ^ (row & 15));
-// X^T tile: chunk (d, c) at d * 4 + (c ^ xt_swz(d)).  The WAVES waves of the
-// workgroup share the tile's 1024 + 1024 chunk loads and its 32 labels.
+// What a lane loads of each tile.  X tile: 16-byte chunk (row, c) at chunk
+// row * 32 + (c ^ (row & 15)); X^T tile: chunk (d, c) at d * 4 + (c ^
+// xt_swz(d)).  The WAVES waves of the workgroup share a tile's 1024 chunk
+// loads and its 32 labels.  The lane's part of an address is the same for
+// every tile and is kept (it was some 130 integer instructions a tile).
 template <int WAVES>
-__device__ inline void stage_tile(const __bf16* X, const __bf16* Xt,
-                                  const float* y, int n_obs, int n0,
-                                  __bf16* xs, __bf16* xts, float* ys, int w,
-                                  int l) {
-  constexpr int U = 16 / WAVES;      // 1 KiB chunk rows per wave and matrix
-  constexpr int YL = kMRows / WAVES; // labels per wave
-  w = __builtin_amdgcn_readfirstlane(w);
+struct TileLoads {
+  static constexpr int U = 16 / WAVES;       // 1 KiB chunk rows per wave
+  static constexpr int YL = kMRows / WAVES;  // labels per wave
+  int w, l;
+  uint32_t xoff[U];  // within a tile of X
+  uint64_t xt0;      // this lane's first chunk of tile 0 of X^T
+  size_t xt_step;    // bytes of 16 rows of X^T
+  __device__ TileLoads(const __bf16* Xt, int n_obs, int wave, int lane)
+      : w(__builtin_amdgcn_readfirstlane(wave)), l(lane) {
 #pragma unroll
-  for (int u = 0; u < U; ++u) {
-    const int q = (w * U + u) * 64 + l;
-    const int row = q >> 5, c = (q & 31) ^ (row & 15);
-    lds_dma16(X + (size_t)(n0 + row) * kMD + c * 8,
-              (char*)xs + (size_t)(w * U + u) * 1024);
+    for (int u = 0; u < U; ++u) {
+      const int q = (w * U + u) * 64 + l;
+      const int row = q >> 5, c = (q & 31) ^ (row & 15);
+      xoff[u] = (uint32_t)(row * kMD + c * 8) * 2;
+    }
+    // rows d = 16 (w U + u) + l / 4: the swizzle repeats every 16
+    const int d = w * U * 16 + (l >> 2), c = (l & 3) ^ xt_swz(l >> 2);
+    xt0 = (uint64_t)(Xt + (size_t)d * n_obs + c * 8);
+    xt_step = (size_t)n_obs * 32;
   }
+  __device__ void x(const __bf16* X, int n0, __bf16* xs) const {
+    const __bf16* g = X + (size_t)n0 * kMD;
 #pragma unroll
-  for (int u = 0; u < U; ++u) {
-    const int q = (w * U + u) * 64 + l;
-    const int d = q >> 2, c = (q & 3) ^ xt_swz(d);
-    lds_dma16(Xt + (size_t)d * n_obs + n0 + c * 8,
-              (char*)xts + (size_t)(w * U + u) * 1024);
+    for (int u = 0; u < U; ++u)
+      lds_dma16(g, xoff[u], (char*)xs + (w * U + u) * 1024);
   }
-  if (l < YL) lds_dma4(y + n0 + w * YL + l, ys + w * YL);
-}
+  __device__ void xt(int n0, __bf16* xts) const {
+    const uint64_t g = xt0 + (size_t)n0 * 2;
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      lds_dma16((const void*)(g + u * xt_step),
+                (char*)xts + (w * U + u) * 1024);
+  }
+  __device__ void labels(const float* y, int n0, float* ys) const {
+    if (l < YL) lds_dma4(y + n0 + w * YL, l * 4, ys + w * YL);
+  }
+};
 
-// s_waitcnt immediate that waits until at most n vector-memory loads of
-// this wave are outstanding (expcnt and lgkmcnt left at their maxima).
-template <int N>
-constexpr int vmcnt_imm() {
-  static_assert(N >= 0 && N < 16, "vmcnt field");
-  return 0xF70 | N;
-}
-
-// Partial gradient (and optionally partial Bernoulli log-likelihood) of the
-// chains [16*WAVES*blockIdx.x, +16*WAVES) over rows
-// [blockIdx.y*rows_per_split, +rows), 16 chains per wave.  With 8 waves
-// (128 chains) every staged tile serves twice the chains of the 4-wave
-// layout, halving the X and X^T bytes staged per gradient; the workgroup
-// then takes one CU (84 KiB of LDS) with the same 8 waves per CU.
+// Partial gradient (and with LL the partial Bernoulli log-likelihood, which a
+// trajectory's last gradient needs) of the chains [32*WAVES*blockIdx.x,
+// +32*WAVES) over rows [blockIdx.y*rows_per_split, +rows), 32 chains per wave,
+// one wave per SIMD (its coefficients and gradients take 256 registers).
+//
+// What bounds it: the matrix unit at the clock the card holds under it.
+// 32x32x16 MFMAs run at 2.23 PFLOP/s here by themselves, 16x16x32 ones (16
+// chains per wave, the layout before) at no more than 1.66, and beside those
+// every VALU instruction adds its whole issue time, while a 32x32x16 hides
+// about four.  So the kernel runs ahead: a step takes the logits of tile t + 2,
+// the residuals of tile t + 1 and the gradient of tile t, which do not depend
+// on each other, two residuals beside every eight products.  65536 x 256, 4096
+// chains (both products with hi and lo parts, 550 GFLOP): 515 -> 470 us, 1.17
+// PFLOP/s, where a large BF16 matrix product reaches 1.13; the matrix unit was
+// busy for 47% of the cycles and is for 60%, at a clock that falls from 2.0 to
+// 1.9 GHz, so that other orders of the same instructions measured the same and
+// fewer instructions less.  An HMC transition, L = 20: 10.59 -> 9.66 ms; of
+// 8192 rows and 64 chains 421 -> 412 us.  The sums are the same bit for bit.
+//
 // Tiles of 32 rows of X and X^T go straight from memory to LDS (no
-// registers) into one of two buffers while the previous tile is used, so a
-// tile's load latency hides behind the previous tile's MFMAs.  LDS layouts
-// (16-byte chunks, XOR-swizzled so that the MFMA fragment reads of 16 rows
-// hit distinct banks): X tile chunk (row, c) at row * 32 + (c ^ (row & 15)),
-// X^T tile chunk (d, c) at d * 4 + (c ^ xt_swz(d)).  Each lane writes its
-// four consecutive residual rows as one 8-byte store (R pitch 40 bf16 keeps
-// those stores and the 16-byte fragment reads free of bank conflicts).
-template <int WAVES>
-__global__ void __launch_bounds__(64 * WAVES, 8 / WAVES)
+// registers).  X is staged two tiles ahead of X^T, each in two buffers, and one
+// barrier a step serves both as "the loads of the last step have landed" and
+// "every wave has left the buffers that this step's loads overwrite".
+// LDS layouts (16-byte chunks, XOR-swizzled so that the MFMA fragment reads of
+// eight consecutive rows hit distinct banks): X tile chunk (row, c) at row * 32
+// + (c ^ (row & 15)), X^T tile chunk (d, c) at d * 4 + (c ^ xt_swz(d)).  Each
+// lane writes four consecutive residual rows as one 8-byte store (R pitch 40
+// bf16 keeps those stores and the 16-byte fragment reads free of conflicts).
+template <int WAVES, bool LL>
+__global__ void __launch_bounds__(64 * WAVES, 1)
     glm_grad_mfma(const __bf16* __restrict__ X, const __bf16* __restrict__ Xt,
                   const float* __restrict__ y, int n_obs,
                   const __bf16* __restrict__ Bhi,
                   const __bf16* __restrict__ Blo, int n_chains,
                   int rows_per_split, float* __restrict__ out_g,
                   float* __restrict__ out_ll) {
-  __shared__ __align__(1024) __bf16 xs0[kMRows * kMD];
-  __shared__ __align__(1024) __bf16 xs1[kMRows * kMD];
-  __shared__ __align__(1024) __bf16 xts0[kMD * kMRows];
-  __shared__ __align__(1024) __bf16 xts1[kMD * kMRows];
-  constexpr int CH = 16 * WAVES;  // chains of the workgroup
+  constexpr int kTile = kMRows * kMD;
+  constexpr int KB = kMD / 32;     // 32-column blocks
+  constexpr int NT = kMD / 32;     // 32-coefficient gradient tiles
+  static_assert(KB == NT, "one block of each in a scheduling region");
+  constexpr int CH = 32 * WAVES;   // chains of the workgroup
+  __shared__ __align__(1024) __bf16 xs[2 * kTile];
+  __shared__ __align__(1024) __bf16 xts[2 * kTile];
   __shared__ __align__(16) __bf16 rs[2 * CH * kRPitch];
-  __shared__ __align__(16) float ys0[kMRows];
-  __shared__ __align__(16) float ys1[kMRows];
+  __shared__ __align__(16) float ys[2 * kMRows];
   const int tid = threadIdx.x;
-  const int w = tid >> 6, l = tid & 63, m = l & 15, g = l >> 4;
-  const int c0 = blockIdx.x * CH + 16 * w;
-  bf16x8 bh[kMD / 32], bl[kMD / 32];
+  const int w = tid >> 6, l = tid & 63, m = l & 31, h = l >> 5;
+  const int c0 = blockIdx.x * CH + 32 * w;
+  const int r0 = blockIdx.y * rows_per_split;
+  const int r1 = min(n_obs, r0 + rows_per_split);
+  const int tiles = (r1 - r0) / kMRows;
+  const TileLoads<WAVES> load(Xt, n_obs, w, l);
+  if (tiles > 0) {
+    load.x(X, r0, xs);
+    load.labels(y, r0, ys);
+    load.xt(r0, xts);
+    if (tiles > 1) {
+      load.x(X, r0 + kMRows, xs + kTile);
+      load.labels(y, r0 + kMRows, ys + kMRows);
+    }
+  }
+  // coefficients of chain m, columns 16 k + 8 h + [0, 8): 1 KiB per load
+  bf16x8 bh[2 * KB], bl[2 * KB];
 #pragma unroll
-  for (int ks = 0; ks < kMD / 32; ++ks) {
-    const size_t off = (size_t)(c0 + m) * kMD + 32 * ks + 8 * g;
-    bh[ks] = *(const bf16x8*)(Bhi + off);
-    bl[ks] = *(const bf16x8*)(Blo + off);
+  for (int k = 0; k < 2 * KB; ++k) {
+    const size_t off = coef_index(c0 + m, 16 * k + 8 * h);
+    bh[k] = *(const bf16x8*)(Bhi + off);
+    bl[k] = *(const bf16x8*)(Blo + off);
   }
   // keep the fragments in registers (not re-read from memory per tile,
   // whose waits would also wait for the tile loads in flight)
 #pragma unroll
-  for (int ks = 0; ks < kMD / 32; ++ks) asm volatile("" : "+v"(bh[ks]), "+v"(bl[ks]));
-  f32x4 acc[kMD / 16];
+  for (int k = 0; k < 2 * KB; ++k) asm volatile("" : "+v"(bh[k]), "+v"(bl[k]));
+  f32x16 acc[NT];
 #pragma unroll
-  for (int nt = 0; nt < kMD / 16; ++nt) acc[nt] = f32x4{0.f, 0.f, 0.f, 0.f};
-  float lls = 0.f;
-  const bool want_ll = out_ll != nullptr;
-  const int r0 = blockIdx.y * rows_per_split;
-  const int r1 = min(n_obs, r0 + rows_per_split);
-  __bf16* rh_w = rs + (16 * w) * kRPitch;
-  __bf16* rl_w = rs + CH * kRPitch + (16 * w) * kRPitch;
+  for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[nt][r] = 0.f;
+  // log-likelihood of the lane's rows, kept as the sums of rows 4 h + [0, 4)
+  // (mod 16) and 8 + 4 h + [0, 4) (mod 16)
+  float lls[2] = {0.f, 0.f};
+  __bf16* rh_w = rs + (32 * w + m) * kRPitch;
+  __bf16* rl_w = rh_w + CH * kRPitch;
 
-  auto compute = [&](const __bf16* xs, const __bf16* xts, const float* ys) {
-    f32x4 s0 = f32x4{0.f, 0.f, 0.f, 0.f}, s1 = s0;
+  // row m of a tile, 16-byte chunk 2 k + h, which sits at (2 k + h) ^ (m % 16)
+  // = 16 (k / 8) + (2 (k % 8) + h) ^ (m % 16): eight lane addresses, the rest
+  // are constants
+  int xo[8];
 #pragma unroll
-    for (int ks = 0; ks < kMD / 32; ++ks) {
-      const int c = 4 * ks + g;
-      const bf16x8 a0 = *(const bf16x8*)&xs[(m * 32 + (c ^ m)) * 8];
-      const bf16x8 a1 = *(const bf16x8*)&xs[((16 + m) * 32 + (c ^ m)) * 8];
-      s0 = mfma16(a0, bh[ks], s0);
-      s1 = mfma16(a1, bh[ks], s1);
-      s0 = mfma16(a0, bl[ks], s0);
-      s1 = mfma16(a1, bl[ks], s1);
+  for (int b = 0; b < 8; ++b) xo[b] = (m * 32 + ((2 * b + h) ^ (m & 15))) * 8;
+  auto x_frag = [&](const __bf16* x, int k) {
+    return *(const bf16x8*)&x[xo[k & 7] + 16 * (k >> 3) * 8];
+  };
+  uint32_t xo_t[2];
+#pragma unroll
+  for (int k = 0; k < 2; ++k)
+    xo_t[k] = (m * 4 + ((2 * k + h) ^ xt_swz(m))) * 16;
+  // residual (and log-likelihood) of one logit
+  auto residual = [&](float sv, float yv, float& ll) {
+    const float e = __expf(-fabsf(sv));
+    const float inv = recip_1p(e);
+    const float sig = sv >= 0.f ? inv : e * inv;
+    if (LL) {
+      const float sp_abs = log1p_unit(e);
+      const float sp_pos = sp_abs + fmaxf(sv, 0.f);
+      const float sp_neg = sp_abs + fmaxf(-sv, 0.f);
+      const float w0 = 1.f - yv;
+      ll += (w0 == 0.f ? 0.f : -sp_pos * w0) + (yv == 0.f ? 0.f : -sp_neg * yv);
     }
+    return yv - sig;
+  };
+  // residuals of the tile behind the logits, and the fragments the gradient
+  // reads: chain m, rows 16 k + 8 h + [0, 8)
+  bf16x8 ah0, ah1, al0, al1;
+  f32x16 s;
+  // one step: S logits of the tile in xn (into s), R residuals of the tile
+  // whose logits s holds, G gradient of the tile in xt whose residuals are in
+  // ah and al.  The three are independent; the scheduling barriers keep a
+  // block's fragment reads one block ahead of its products and two residuals
+  // beside each block of eight.
+  auto step = [&](auto do_s, auto do_r, auto do_g, const __bf16* xn,
+                  const __bf16* xt, const float* yt) {
+    constexpr bool S = decltype(do_s)::value, R = decltype(do_r)::value,
+                   G = decltype(do_g)::value;
+    const uint32_t xt_base = G ? lds_addr((void*)xt) : 0;
+    f32x16 n;
 #pragma unroll
-    for (int mt = 0; mt < 2; ++mt) {
-      bf16x4 hv, lv;
+    for (int r = 0; r < 16; ++r) n[r] = 0.f;
+    // chunks 2 k + h of X^T row 32 nt + m: two lane addresses (opaque, or the
+    // compiler keeps and adds sixteen)
+    uint32_t xa[2];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int row = 16 * mt + 4 * g + i;
-        const float sv = mt ? s1[i] : s0[i];
-        const float yv = ys[row];
-        const float e = __expf(-fabsf(sv));
-        const float inv = recip_1p(e);
-        const float sig = sv >= 0.f ? inv : e * inv;
-        const float r = yv - sig;
-        if (want_ll) {
-          const float sp_abs = log1p_unit(e);
-          const float sp_pos = sp_abs + fmaxf(sv, 0.f);
-          const float sp_neg = sp_abs + fmaxf(-sv, 0.f);
-          const float w0 = 1.f - yv;
-          lls += (w0 == 0.f ? 0.f : -sp_pos * w0) + (yv == 0.f ? 0.f : -sp_neg * yv);
+    for (int k = 0; k < 2; ++k) {
+      xa[k] = xt_base + xo_t[k];
+      asm volatile("" : "+v"(xa[k]));
+    }
+    auto xt_frag = [&](int nt, int k) {
+      return *(lds_bf16x8*)(uintptr_t)(xa[k] + 2048 * nt);
+    };
+    uint32_t hv = 0, lv = 0;
+    f32x4 yv;
+    bf16x8 a0, a1, t0, t1;
+    if (S) {
+      a0 = x_frag(xn, 0);
+      a1 = x_frag(xn, 1);
+    }
+    if (G) {
+      t0 = xt_frag(0, 0);
+      t1 = xt_frag(0, 1);
+    }
+    if (R) yv = *(const f32x4*)&yt[4 * h];
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb) {
+      bf16x8 b0, b1, u0, u1;
+      f32x4 yn;
+      if (S && kb + 1 < KB) {
+        b0 = x_frag(xn, 2 * kb + 2);
+        b1 = x_frag(xn, 2 * kb + 3);
+      }
+      if (G && kb + 1 < NT) {
+        u0 = xt_frag(kb + 1, 0);
+        u1 = xt_frag(kb + 1, 1);
+      }
+      const int q = kb >> 1;  // rows 8 q + 4 h + [0, 4)
+      if (R && (kb & 1) && kb + 1 < KB)
+        yn = *(const f32x4*)&yt[8 * q + 8 + 4 * h];
+      if (S) n = mfma32(a0, bh[2 * kb], n);
+      if (G) acc[kb] = mfma32(ah0, t0, acc[kb]);
+      if (S) n = mfma32(a1, bh[2 * kb + 1], n);
+      if (G) acc[kb] = mfma32(ah1, t1, acc[kb]);
+      if (S) n = mfma32(a0, bl[2 * kb], n);
+      if (G) acc[kb] = mfma32(al0, t0, acc[kb]);
+      if (S) n = mfma32(a1, bl[2 * kb + 1], n);
+      if (G) acc[kb] = mfma32(al1, t1, acc[kb]);
+      if (R) {
+        const int i = 2 * (kb & 1);
+        const float ra = residual(s[4 * q + i], yv[i], lls[q & 1]);
+        const float rb = residual(s[4 * q + i + 1], yv[i + 1], lls[q & 1]);
+        const uint32_t hi = pack_bf16(ra, rb);
+        const uint32_t lo = pack_bf16(ra - __uint_as_float(hi << 16),
+                                      rb - __uint_as_float(hi & 0xffff0000u));
+        if (kb & 1) {
+          *(uint2*)&rh_w[8 * q + 4 * h] = make_uint2(hv, hi);
+          *(uint2*)&rl_w[8 * q + 4 * h] = make_uint2(lv, lo);
         }
-        hv[i] = (__bf16)r;
-        lv[i] = (__bf16)(r - (float)hv[i]);
+        hv = hi;
+        lv = lo;
       }
-      *(bf16x4*)&rh_w[m * kRPitch + 16 * mt + 4 * g] = hv;
-      *(bf16x4*)&rl_w[m * kRPitch + 16 * mt + 4 * g] = lv;
+      if (S) {
+        a0 = b0;
+        a1 = b1;
+      }
+      if (G) {
+        t0 = u0;
+        t1 = u1;
+      }
+      if (R && (kb & 1)) yv = yn;
+      __builtin_amdgcn_sched_barrier(0);
     }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    const bf16x8 ah = *(const bf16x8*)&rh_w[m * kRPitch + 8 * g];
-    const bf16x8 al = *(const bf16x8*)&rl_w[m * kRPitch + 8 * g];
-#pragma unroll
-    for (int nt0 = 0; nt0 < kMD / 16; nt0 += 4) {
-      bf16x8 b[4];
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const int d = 16 * (nt0 + u) + m;
-        b[u] = *(const bf16x8*)&xts[(d * 4 + (g ^ xt_swz(d))) * 8];
-      }
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        acc[nt0 + u] = mfma16(ah, b[u], acc[nt0 + u]);
-        acc[nt0 + u] = mfma16(al, b[u], acc[nt0 + u]);
-      }
+    if (S) s = n;
+    if (R) {
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      ah0 = *(const bf16x8*)&rh_w[8 * h];
+      ah1 = *(const bf16x8*)&rh_w[16 + 8 * h];
+      al0 = *(const bf16x8*)&rl_w[8 * h];
+      al1 = *(const bf16x8*)&rl_w[16 + 8 * h];
     }
   };
-  // tiles of this split, two per round (buffers 0 and 1): the next tile's
-  // LPW loads per wave are issued, then the wave waits until only those are
-  // outstanding (vmcnt(LPW)), i.e. until its loads of the current tile have
-  // landed; the barrier makes every wave's part visible
-  constexpr int LPW = 2 * (16 / WAVES) + 1;
-  if (r0 < r1) stage_tile<WAVES>(X, Xt, y, n_obs, r0, xs0, xts0, ys0, w, l);
-  for (int n0 = r0; n0 < r1; n0 += 2 * kMRows) {
-    const int n1 = n0 + kMRows;
-    if (n1 < r1) {
-      stage_tile<WAVES>(X, Xt, y, n_obs, n1, xs1, xts1, ys1, w, l);
-      __builtin_amdgcn_s_waitcnt(vmcnt_imm<LPW>());  // tile n0 has landed
+  using Yes = std::true_type;
+  using No = std::false_type;
+  auto landed = [&] {
+    __builtin_amdgcn_s_waitcnt(0xF70);  // this wave's tile loads (vmcnt)
+    __syncthreads();
+  };
+  // Step t: logits of tile t + 2, residuals of t + 1, gradient of t.  Buffer
+  // j & 1 holds tile j of X, X^T and y; the loads a step issues replace what
+  // the step before it read: X of t + 3, X^T of t + 1, y of t + 2.
+  if (tiles > 0) {
+    landed();
+    step(Yes{}, No{}, No{}, xs, nullptr, nullptr);
+    if (tiles > 1) {
+      landed();
+      if (tiles > 2) load.x(X, r0 + 2 * kMRows, xs);
+      step(Yes{}, Yes{}, No{}, xs + kTile, nullptr, ys);
     } else {
-      __builtin_amdgcn_s_waitcnt(vmcnt_imm<0>());
+      step(No{}, Yes{}, No{}, nullptr, nullptr, ys);
     }
-    __syncthreads();
-    compute(xs0, xts0, ys0);
-    __syncthreads();
-    if (n1 >= r1) break;
-    const int n2 = n1 + kMRows;
-    if (n2 < r1) {
-      stage_tile<WAVES>(X, Xt, y, n_obs, n2, xs0, xts0, ys0, w, l);
-      __builtin_amdgcn_s_waitcnt(vmcnt_imm<LPW>());
-    } else {
-      __builtin_amdgcn_s_waitcnt(vmcnt_imm<0>());
-    }
-    __syncthreads();
-    compute(xs1, xts1, ys1);
-    __syncthreads();
+  }
+  for (int t = 0; t + 2 < tiles; ++t) {
+    landed();
+    const int n0 = r0 + t * kMRows;
+    const int b = t & 1, o = b ^ 1;
+    if (t + 3 < tiles) load.x(X, n0 + 3 * kMRows, xs + o * kTile);
+    load.xt(n0 + kMRows, xts + o * kTile);
+    load.labels(y, n0 + 2 * kMRows, ys + b * kMRows);
+    step(Yes{}, Yes{}, Yes{}, xs + b * kTile, xts + b * kTile,
+         ys + o * kMRows);
+  }
+  if (tiles > 1) {
+    landed();
+    const int b = tiles & 1, o = b ^ 1;
+    load.xt(r0 + (tiles - 1) * kMRows, xts + o * kTile);
+    step(No{}, Yes{}, Yes{}, nullptr, xts + b * kTile, ys + o * kMRows);
+  }
+  if (tiles > 0) {
+    if (tiles > 1) landed();
+    step(No{}, No{}, Yes{}, nullptr, xts + ((tiles - 1) & 1) * kTile, nullptr);
   }
   float* og = out_g + ((size_t)blockIdx.y * n_chains + c0) * kMD;
 #pragma unroll
-  for (int nt = 0; nt < kMD / 16; ++nt)
+  for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
-    for (int i = 0; i < 4; ++i) og[(size_t)(4 * g + i) * kMD + 16 * nt + m] = acc[nt][i];
-  if (want_ll) {
-    lls += __shfl_xor(lls, 16);
-    lls += __shfl_xor(lls, 32);
-    if (g == 0) out_ll[(size_t)blockIdx.y * n_chains + c0 + m] = lls;
+    for (int r = 0; r < 16; ++r)
+      og[(size_t)(8 * (r >> 2) + 4 * h + (r & 3)) * kMD + 32 * nt + m] =
+          acc[nt][r];
+  if (LL) {
+    const float p = lls[0] + __shfl_xor(lls[0], 32);
+    const float q = lls[1] + __shfl_xor(lls[1], 32);
+    if (h == 0) out_ll[(size_t)blockIdx.y * n_chains + c0 + m] = p + q;
   }
 }
 // ---------------------------------------------------------------- per chain
@@ -271,8 +425,9 @@ __global__ void mfma_prepare(hipmc_glm_hmc_args a) {
   if (i >= (size_t)a.n_chains * kMD) return;
   __bf16 hi, lo;
   split_bf16(a.state[i], hi, lo);
-  ((__bf16*)a.ws_b)[i] = hi;
-  ((__bf16*)a.ws_b)[(size_t)a.n_chains * kMD + i] = lo;
+  const size_t o = coef_index((int)(i / kMD), (int)(i % kMD));
+  ((__bf16*)a.ws_b)[o] = hi;
+  ((__bf16*)a.ws_b)[(size_t)a.n_chains * kMD + o] = lo;
 }
 
 // Element e of chain c: the split-N partial gradients added in split order,
@@ -348,8 +503,8 @@ __global__ void __launch_bounds__(kMD) mfma_chain_step(hipmc_glm_hmc_args a,
   const size_t row = (size_t)c * kMD;
   float* q = a.ws_q + row;
   float* p = a.ws_p + row;
-  __bf16* bh = (__bf16*)a.ws_b + row;
-  __bf16* bl = (__bf16*)a.ws_b + (size_t)a.n_chains * kMD + row;
+  __bf16* bh = (__bf16*)a.ws_b + coef_index(c, e);
+  __bf16* bl = bh + (size_t)a.n_chains * kMD;
   if (mode == 3) {
     const float qv = a.state[row + e];
     a.grad[row + e] = reduce_grad(a, c, e, qv, inv_ps2);
@@ -383,8 +538,8 @@ __global__ void __launch_bounds__(kMD) mfma_chain_step(hipmc_glm_hmc_args a,
     q[e] = qv;
     __bf16 hi, lo;
     split_bf16(qv, hi, lo);
-    bh[e] = hi;
-    bl[e] = lo;
+    *bh = hi;
+    *bl = lo;
     red[0][e] = (double)pv0 * (double)pv0;
     __syncthreads();
     if (first) {
@@ -402,8 +557,8 @@ __global__ void __launch_bounds__(kMD) mfma_chain_step(hipmc_glm_hmc_args a,
     q[e] = qn;
     __bf16 hi, lo;
     split_bf16(qn, hi, lo);
-    bh[e] = hi;
-    bl[e] = lo;
+    *bh = hi;
+    *bl = lo;
     return;
   }
   // mode 2: last kick, un-kick, kinetic energy, log-prob, MH accept

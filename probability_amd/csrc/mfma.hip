@@ -76,7 +76,10 @@ int launch_glm_hmc(const hipmc_glm_hmc_args* a, hipStream_t s) {
   if (n_split != a->n_split)
     return fail(HIPMC_E_INVALID, "glm_hmc: n_split leaves an empty split; use fewer");
   // 128 chains per workgroup when the chain count allows (each staged tile
-  // then serves 8 waves), else 64
+  // then serves 4 waves: a transition of 4096 rows, 1024 chains, L = 20 takes
+  // 566 us), else 64 (four waves for those, each with half the coefficients,
+  // took 12% to 30% longer than two, from 32768 rows on: the logits are then
+  // computed twice)
   const bool wide = a->n_chains % (2 * kMChains) == 0;
   const dim3 ggrid(a->n_chains / (wide ? 2 * kMChains : kMChains), n_split);
   const dim3 cgrid(a->n_chains);
@@ -84,16 +87,18 @@ int launch_glm_hmc(const hipmc_glm_hmc_args* a, hipStream_t s) {
     const __bf16* bh = (const __bf16*)a->ws_b;
     const __bf16* bl = bh + (size_t)a->n_chains * kMD;
     float* oll = ll ? a->ws_ll : nullptr;
+    auto launch = [&](auto kernel, int threads) {
+      hipLaunchKernelGGL(kernel, ggrid, dim3(threads), 0, s,
+                         (const __bf16*)a->x_bf16, (const __bf16*)a->xt_bf16,
+                         a->y, a->n_obs, bh, bl, a->n_chains, rps, a->ws_g,
+                         oll);
+    };
     if (wide)
-      hipLaunchKernelGGL(glm_grad_mfma<8>, ggrid, dim3(512), 0, s,
-                         (const __bf16*)a->x_bf16, (const __bf16*)a->xt_bf16,
-                         a->y, a->n_obs, bh, bl, a->n_chains, rps, a->ws_g,
-                         oll);
+      ll ? launch(glm_grad_mfma<4, true>, 256)
+         : launch(glm_grad_mfma<4, false>, 256);
     else
-      hipLaunchKernelGGL(glm_grad_mfma<4>, ggrid, dim3(256), 0, s,
-                         (const __bf16*)a->x_bf16, (const __bf16*)a->xt_bf16,
-                         a->y, a->n_obs, bh, bl, a->n_chains, rps, a->ws_g,
-                         oll);
+      ll ? launch(glm_grad_mfma<2, true>, 128)
+         : launch(glm_grad_mfma<2, false>, 128);
   };
   if (a->want_grad_only) {
     const size_t ne = (size_t)a->n_chains * kMD;
