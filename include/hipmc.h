@@ -477,6 +477,23 @@ int hipmc_mh_accept(int32_t dtype, int32_t n_chains, int32_t dim_stride,
                     void* grad, void* out_log_accept_ratio,
                     uint8_t* out_is_accepted, uint64_t stream);
 
+/* Copies of up to HIPMC_MAX_COPY_BLOCKS strided blocks of `rows` x `cols`
+ * elements (4 or 8 bytes each) in one launch: what packs state parts into the
+ * flat layout, and with a row mask what selects an accepted chain's values:
+ * dst[r, c] = mask == NULL || mask[r] ? src[r, c] : alt[r, c].  Strides are in
+ * elements; dst's columns are adjacent. */
+#define HIPMC_MAX_COPY_BLOCKS 16
+typedef struct hipmc_copy_block {
+  const void* src;
+  const void* alt;
+  void* dst;
+  int64_t src_row, src_col, alt_row, alt_col, dst_row;
+  int32_t rows, cols;
+} hipmc_copy_block;
+int hipmc_copy_blocks(int32_t elem_size, int32_t n,
+                      const hipmc_copy_block* blocks, const uint8_t* mask,
+                      uint64_t stream);
+
 /* Elementwise bijector on x [n_rows, dim_stride] per the problem's bijector
  * ranges: direction 0 = forward, 1 = inverse.  Row r is chain
  * (chain_period > 0 ? r % chain_period : r) of chain_problem (a trace of

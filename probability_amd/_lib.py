@@ -30,7 +30,7 @@ EXPORTED_SYMBOLS = (
     'hipmc_seed_salt', 'hipmc_philox_host', 'hipmc_hmc_run',
     'hipmc_leapfrog_run', 'hipmc_nuts_run', 'hipmc_target_eval',
     'hipmc_da_update', 'hipmc_simple_step_update', 'hipmc_mh_accept',
-    'hipmc_bijector', 'hipmc_draws', 'hipmc_moments_update',
+    'hipmc_bijector', 'hipmc_copy_blocks', 'hipmc_draws', 'hipmc_moments_update',
     'hipmc_variance_update', 'hipmc_glm_hmc_run_noalloc',
     'hipmc_effective_sample_size', 'hipmc_potential_scale_reduction',
     'hipmc_glm_tile_plan', 'hipmc_glm_tile_eval',
@@ -169,6 +169,7 @@ def lib():
           _vp, _vp, _vp, _u64]
       l.hipmc_glm_tile_hmc_run.argtypes = [ctypes.POINTER(RunArgs), _i32, _i32,
                                            _i32, _vp, _i64, _u64]
+      l.hipmc_copy_blocks.argtypes = [_i32, _i32, _vp, _vp, _u64]
       l.hipmc_bijector.argtypes = [_i32, _vp, _vp, _i32, _i32, _i32, _i32,
                                    _vp, _vp, _u64]
       l.hipmc_draws.argtypes = [_i32, _i32, _vp, _i32, _i32, _i32, _i32, _i32,
@@ -207,7 +208,35 @@ def ptr(t):
 
 
 def stream_handle(device=None):
+  """hipStream_t of the device's current stream (current_stream() without the
+  Stream object, which takes 2 us of every launch)."""
+  if device is None or (isinstance(device, torch.device) and
+                        device.type == 'cuda'):
+    index = device.index if device is not None else None
+    current = torch.cuda.current_device()  # initialises the runtime
+    return torch._C._cuda_getCurrentRawStream(
+        current if index is None else index)
   return torch.cuda.current_stream(device).cuda_stream
+
+
+MAX_COPY_BLOCKS = 16
+
+
+def copy_blocks(blocks, elem_size, device, mask=None):
+  """hipmc_copy_blocks of [(src, alt, dst, dst_row)]: src and alt (None
+  without a mask) are 2-D tensors of equal shape, dst the address of the
+  result, whose rows are `dst_row` elements apart."""
+  words = []
+  for src, alt, dst, dst_row in blocks:
+    rows, cols = src.shape
+    sr, sc = src.stride()
+    ar, ac = alt.stride() if alt is not None else (0, 0)
+    words += (src.data_ptr(), 0 if alt is None else alt.data_ptr(),
+              dst, sr, sc, ar, ac, dst_row, rows | cols << 32)
+  raw = (_i64 * len(words))(*words)
+  check(lib().hipmc_copy_blocks(elem_size, len(blocks), raw,
+                                None if mask is None else mask.data_ptr(),
+                                stream_handle(device)))
 
 
 def glm_waves_per_chain(max_rows_times_cols):

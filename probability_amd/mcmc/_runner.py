@@ -9,7 +9,9 @@ import torch
 
 from probability_amd import _lib
 from probability_amd import glm_tile
+from probability_amd import targets as targets_lib
 from probability_amd import tuning
+from probability_amd.mcmc.internal import util as mcmc_util
 
 _OUT_FIELDS = ('out_log_accept_ratio', 'out_leapfrogs', 'out_is_accepted',
                'out_reach_max_depth', 'out_has_divergence', 'out_energy',
@@ -28,6 +30,11 @@ def step_tensor(step_size, dtype, device):
         raise NotImplementedError(
             'per-part step sizes that differ are not built into the kernels')
     step_size = first
+  # a Python number is filled in on the device: the copy of a pageable tensor
+  # waits for the stream's earlier work
+  if (type(step_size) is float and device.type == 'cuda' and
+      abs(step_size) <= torch.finfo(dtype).max):
+    return torch.full((1,), step_size, dtype=dtype, device=device)
   t = torch.as_tensor(step_size, dtype=dtype)
   return t.to(device).reshape(-1).contiguous()
 
@@ -98,7 +105,34 @@ class Run:
 
 def flat_inputs(spec, parts, tlp, grads):
   """Packs state/grad parts; returns contiguous working copies."""
-  state = spec.pack_state(parts).clone()
-  grad = spec.pack_state(grads).clone()
-  t = tlp.to(device=spec.device, dtype=spec.dtype).reshape(-1).clone()
-  return state, t, grad
+  # tlp has one element per chain in any shape: its own list
+  state, grad, t = targets_lib.pack_states(
+      [(parts, spec.event_shapes), (grads, spec.event_shapes),
+       ([tlp], [()])], spec.dtype, spec.device)
+  return state, t.reshape(-1), grad
+
+
+def choose_rows(accepted, proposed, current):
+  """[torch.where(accepted, p, c)] of lists of per-chain tensors, in one
+  launch where they are plain tensors of one type and shape on the current
+  GPU."""
+  n = accepted.numel()
+  first = proposed[0]
+  if (n == 0 or len(proposed) > _lib.MAX_COPY_BLOCKS or not first.is_cuda or
+      first.device.index != torch.cuda.current_device() or
+      first.element_size() not in (4, 8) or
+      any(not isinstance(c, torch.Tensor) or c.requires_grad or
+          c.is_neg() or p.is_neg() or
+          c.dtype != first.dtype or p.dtype != first.dtype or
+          c.device != first.device or c.shape != p.shape or
+          p.shape[:accepted.dim()] != accepted.shape or
+          not 0 < p.numel() < 1 << 31 for p, c in zip(proposed, current))):
+    return mcmc_util.choose(accepted, list(proposed), list(current))
+  out = [torch.empty(p.shape, dtype=p.dtype, device=p.device)
+         for p in proposed]
+  blocks = []
+  for p, c, o in zip(proposed, current, out):
+    p = p.reshape(n, -1)
+    blocks.append((p, c.reshape(n, -1), o.data_ptr(), p.shape[1]))
+  _lib.copy_blocks(blocks, first.element_size(), first.device, accepted)
+  return out

@@ -203,7 +203,7 @@ class HamiltonianMonteCarlo(kernel_base.TransitionKernel):
     run.args.num_leapfrog_steps = nsteps
     c, d = state.shape
     lar = run.want('out_log_accept_ratio', (1, c), spec.dtype)
-    is_acc = run.want('out_is_accepted', (1, c), torch.uint8)
+    is_acc = run.want('out_is_accepted', (1, c), torch.bool)
     corr = run.want('out_energy', (1, c), spec.dtype)
     pst = run.want('out_proposed_state', (c, d), spec.dtype)
     ptlp = run.want('out_proposed_tlp', (c,), spec.dtype)
@@ -211,24 +211,26 @@ class HamiltonianMonteCarlo(kernel_base.TransitionKernel):
     p1 = run.want('out_final_momentum', (c, d), spec.dtype)
     run.call_hmc(True)
     cs = tuple(acc.target_log_prob.shape)
-    accepted = is_acc.reshape(cs).bool()
+    accepted = is_acc.reshape(cs)
     proposed_results = acc._replace(
         log_acceptance_correction=corr.reshape(cs),
         target_log_prob=ptlp.reshape(cs),
         grads_target_log_prob=None,
         initial_momentum=spec.unpack_state(p0, cs),
         final_momentum=spec.unpack_state(p1, cs),
-        seed=samplers.split_seed(seed, 2)[0])
+        seed=samplers.first_child(seed))
+    k = len(proposed_results.initial_momentum)
+    chosen = _runner.choose_rows(
+        accepted, [proposed_results.log_acceptance_correction,
+                   *proposed_results.initial_momentum,
+                   *proposed_results.final_momentum],
+        [acc.log_acceptance_correction, *_as_parts(acc.initial_momentum),
+         *_as_parts(acc.final_momentum)])
     new_acc = acc._replace(
-        log_acceptance_correction=torch.where(
-            accepted, proposed_results.log_acceptance_correction,
-            acc.log_acceptance_correction),
+        log_acceptance_correction=chosen[0],
         target_log_prob=tlp.reshape(cs),
         grads_target_log_prob=spec.unpack_state(grad, cs),
-        initial_momentum=mcmc_util.choose(
-            accepted, proposed_results.initial_momentum, acc.initial_momentum),
-        final_momentum=mcmc_util.choose(
-            accepted, proposed_results.final_momentum, acc.final_momentum),
+        initial_momentum=chosen[1:1 + k], final_momentum=chosen[1 + k:],
         seed=[])
     results = mh.MetropolisHastingsKernelResults(
         accepted_results=new_acc, is_accepted=accepted,
@@ -257,12 +259,12 @@ class HamiltonianMonteCarlo(kernel_base.TransitionKernel):
     c = state.shape[0]
     run = self.mfma_runner(spec, c)
     lar = torch.empty((1, c), dtype=torch.float32, device=spec.device)
-    isacc = torch.empty((1, c), dtype=torch.uint8, device=spec.device)
+    isacc = torch.empty((1, c), dtype=torch.bool, device=spec.device)
     run.run(state, tlp, grad, _runner.step_tensor(step_size, spec.dtype,
                                                   spec.device),
             seed, nsteps, out_lar=lar, out_acc=isacc)
     cs = tuple(acc.target_log_prob.shape)
-    accepted = isacc.reshape(cs).bool()
+    accepted = isacc.reshape(cs)
     new_acc = acc._replace(target_log_prob=tlp.reshape(cs),
                            grads_target_log_prob=spec.unpack_state(grad, cs),
                            seed=[])

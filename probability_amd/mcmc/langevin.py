@@ -174,19 +174,19 @@ class MetropolisAdjustedLangevinAlgorithm(kernel_base.TransitionKernel):
     run.args.num_leapfrog_steps = 1
     c, d = state.shape
     lar = run.want('out_log_accept_ratio', (1, c), spec.dtype)
-    is_acc = run.want('out_is_accepted', (1, c), torch.uint8)
+    is_acc = run.want('out_is_accepted', (1, c), torch.bool)
     corr = run.want('out_energy', (1, c), spec.dtype)
     pst = run.want('out_proposed_state', (c, d), spec.dtype)
     ptlp = run.want('out_proposed_tlp', (c,), spec.dtype)
     run.call_hmc(True)
     cs = tuple(acc.target_log_prob.shape)
-    accepted = is_acc.reshape(cs).bool()
+    accepted = is_acc.reshape(cs)
     # the proposal's gradient is not kept by the fused launch (the accepted
     # chains' gradient is in `grad`)
     proposed = acc._replace(
         log_acceptance_correction=corr.reshape(cs),
         target_log_prob=ptlp.reshape(cs), grads_target_log_prob=None,
-        diffusion_drift=None, seed=samplers.split_seed(seed, 2)[0])
+        diffusion_drift=None, seed=samplers.first_child(seed))
     new_acc = _results(spec, cs, self.step_size, tlp, grad,
                        torch.where(accepted, corr.reshape(cs),
                                    acc.log_acceptance_correction), [])

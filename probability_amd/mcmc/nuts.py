@@ -137,9 +137,9 @@ class NoUTurnSampler(kernel_base.TransitionKernel):
     c = state.shape[0]
     lar = run.want('out_log_accept_ratio', (1, c), spec.dtype)
     lf = run.want('out_leapfrogs', (1, c), torch.int32)
-    acc = run.want('out_is_accepted', (1, c), torch.uint8)
-    rmd = run.want('out_reach_max_depth', (1, c), torch.uint8)
-    div = run.want('out_has_divergence', (1, c), torch.uint8)
+    acc = run.want('out_is_accepted', (1, c), torch.bool)
+    rmd = run.want('out_reach_max_depth', (1, c), torch.bool)
+    div = run.want('out_has_divergence', (1, c), torch.bool)
     energy = run.want('out_energy', (1, c), spec.dtype)
     run.call(_lib.lib().hipmc_nuts_run)
     cs = tuple(pkr.target_log_prob.shape)
@@ -149,9 +149,9 @@ class NoUTurnSampler(kernel_base.TransitionKernel):
         step_size=pkr.step_size,
         log_accept_ratio=lar.reshape(cs),
         leapfrogs_taken=lf.reshape(cs),
-        is_accepted=acc.reshape(cs).bool(),
-        reach_max_depth=rmd.reshape(cs).bool(),
-        has_divergence=div.reshape(cs).bool(),
+        is_accepted=acc.reshape(cs),
+        reach_max_depth=rmd.reshape(cs),
+        has_divergence=div.reshape(cs),
         energy=energy.reshape(cs),
         seed=seed)
     next_parts = spec.unpack_state(state, cs)

@@ -49,9 +49,11 @@ def _update_target_log_prob(kernel, new_target):
 
 def _map_state(spec, bijectors, parts, direction):
   """Elementwise forward (0) / inverse (1) of every part, on the device."""
-  dev_parts = [targets_lib._to_device(p, spec.dtype, spec.device) for p in parts]
-  cs = spec.chain_shape(dev_parts)
-  flat = spec.pack_state(dev_parts)
+  parts = [p if isinstance(p, torch.Tensor)
+           else targets_lib._to_device(p, spec.dtype, spec.device)
+           for p in parts]
+  cs = spec.chain_shape(parts)
+  flat = spec.pack_state(parts)
   out = torch.empty_like(flat)
   _lib.check(_lib.lib().hipmc_bijector(
       _lib.dtype_code(spec.dtype), _lib.ptr(spec.table(bijectors)), None,

@@ -52,6 +52,14 @@ def split_seed(seed, n=2):
   return out
 
 
+def first_child(seed):
+  """split_seed(seed)[0]."""
+  out = np.zeros(2, np.uint32)
+  _lib.check(_lib.lib().hipmc_seed_split(_ptr(sanitize_seed(seed)),
+                                          ctypes.c_uint32(0), _ptr(out)))
+  return out
+
+
 def fold_in(seed, t):
   """Seed of step t of a sampling loop."""
   s = sanitize_seed(seed)

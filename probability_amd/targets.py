@@ -34,10 +34,7 @@ def _to_device(x, dtype, device):
 
 
 def _numel(shape):
-  n = 1
-  for s in shape:
-    n *= int(s)
-  return n
+  return math.prod(shape)
 
 
 class TargetSpec:
@@ -211,25 +208,58 @@ class TransformedTarget(TargetSpec):
 
 def pack_state(parts, event_shapes, dtype, device):
   """List of [chain..., event...] tensors -> [C, dim] contiguous tensor."""
-  flat = []
-  cs = None
-  for p, es in zip(parts, event_shapes):
-    p = _to_device(p, dtype, device)
-    lead = tuple(p.shape[:p.dim() - len(es)])
-    if cs is None:
-      cs = lead
-    elif lead != cs:
-      raise ValueError(f'state parts disagree on chain shape: {lead} vs {cs}')
-    flat.append(p.reshape(_numel(cs), _numel(es)))
-  return torch.cat(flat, dim=1).contiguous()
+  return pack_states([(parts, event_shapes)], dtype, device)[0]
+
+
+def pack_states(lists, dtype, device):
+  """pack_state of several (parts, event_shapes).  On the current GPU one
+  launch copies the parts of all of them, whatever their strides."""
+  out, blocks = [], []
+  for parts, event_shapes in lists:
+    flat = []
+    cs = None
+    for p, es in zip(parts, event_shapes):
+      if isinstance(p, torch.Tensor):
+        p = p.detach().to(device, dtype)
+      else:
+        p = _to_device(p, dtype, device)
+      lead = tuple(p.shape[:p.dim() - len(es)])
+      if cs is None:
+        cs = lead
+      elif lead != cs:
+        raise ValueError(
+            f'state parts disagree on chain shape: {lead} vs {cs}')
+      p = p.reshape(_numel(cs), _numel(es))
+      flat.append(p.resolve_neg() if p.is_neg() else p)
+    if (not flat or not flat[0].is_cuda or
+        flat[0].device.index != torch.cuda.current_device() or
+        len(blocks) + len(flat) > _lib.MAX_COPY_BLOCKS or
+        max(f.numel() for f in flat) >= 1 << 31):
+      out.append(torch.cat(flat, dim=1).contiguous())
+      continue
+    dim = sum(f.shape[1] for f in flat)
+    packed = torch.empty((flat[0].shape[0], dim), dtype=dtype,
+                         device=flat[0].device)
+    dst = packed.data_ptr()
+    for f in flat:
+      blocks.append((f, None, dst, dim))
+      dst += f.shape[1] * dtype.itemsize
+    out.append(packed)
+  if blocks:
+    _lib.copy_blocks(blocks, dtype.itemsize, blocks[0][0].device)
+  return out
 
 
 def unpack_state(flat, chain_shape, event_shapes):
+  """Views of the parts of flat [C, dim] as [chain..., event...] tensors."""
+  cs = tuple(chain_shape)
   out = []
   off = 0
   for es in event_shapes:
     n = _numel(es)
-    out.append(flat[:, off:off + n].reshape(tuple(chain_shape) + tuple(es)))
+    shape = cs + tuple(es)
+    col = flat.narrow(1, off, n)
+    out.append(col if col.shape == shape else col.reshape(shape))
     off += n
   return out
 

@@ -52,10 +52,27 @@ def _load():
   return _table
 
 
+# choices of the loaded table by argument (the table's logarithms take 50 us
+# of every launch otherwise)
+_choices = (None, {})
+
+
 def glm_waves(kind, n_obs, dim, chains, sampler='nuts', dtype=torch.float32):
   """Waves per chain for a GLM launch of `chains` chains of an N x D
   problem: the tuned choice of the nearest measured point, else the rule."""
-  rows = _load().get('glm_waves', {}).get(str(dtype).replace('torch.', ''), [])
+  global _choices
+  table, known = _choices
+  if table is not _load() or len(known) >= 4096:
+    table, known = _choices = (_load(), {})
+  key = (kind, n_obs, dim, chains, sampler, dtype)
+  w = known.get(key)
+  if w is None:
+    w = known[key] = _glm_waves(table, *key)
+  return w
+
+
+def _glm_waves(table, kind, n_obs, dim, chains, sampler, dtype):
+  rows = table.get('glm_waves', {}).get(str(dtype).replace('torch.', ''), [])
   name = 'linear' if kind == _lib.TARGET_LINEAR else 'logistic'
   best, dist = None, None
   for r in rows:
