@@ -355,6 +355,19 @@ int hipmc_leapfrog_run(const hipmc_run_args* args, uint64_t stream);
 /* NUTS for n_iters iterations (per-chain wavefront state machine). */
 int hipmc_nuts_run(const hipmc_run_args* args, uint64_t stream);
 
+/* hipmc_nuts_run whose chains go to the blocks that are ready for one, where
+ * a chain has a block of its own and there are more chains than fit the GPU
+ * at once (elsewhere it is hipmc_nuts_run).  queue: device,
+ * [HIPMC_QUEUE_WORDS], zero before the first launch and left zero by each; a
+ * queue serves one launch at a time.  order: device, [9 + n_chains], the
+ * starts of eight lists and their common end, then the chains (each once) in
+ * the order in which they are taken; XCD x's blocks take list x first.  NULL:
+ * the eighths of 0, 1, ...  The results are those of hipmc_nuts_run bit for
+ * bit. */
+#define HIPMC_QUEUE_WORDS 16
+int hipmc_nuts_run_queued(const hipmc_run_args* args, int32_t* queue,
+                          const int32_t* order, uint64_t stream);
+
 /* target log-prob and gradient at `x` [n_chains, dim_stride]. */
 int hipmc_target_eval(int32_t dtype, int32_t target_kind,
                       const hipmc_problem* problems,

@@ -28,7 +28,8 @@ EXPORTED_SYMBOLS = (
     'hipmc_sizeof_run_args', 'hipmc_sizeof_stream',
     'hipmc_sizeof_glm_hmc_args', 'hipmc_glm_hmc_run', 'hipmc_seed_split', 'hipmc_seed_fold_in',
     'hipmc_seed_salt', 'hipmc_philox_host', 'hipmc_hmc_run',
-    'hipmc_leapfrog_run', 'hipmc_nuts_run', 'hipmc_target_eval',
+    'hipmc_leapfrog_run', 'hipmc_nuts_run', 'hipmc_nuts_run_queued',
+    'hipmc_target_eval',
     'hipmc_da_update', 'hipmc_simple_step_update', 'hipmc_mh_accept',
     'hipmc_bijector', 'hipmc_copy_blocks', 'hipmc_draws', 'hipmc_moments_update',
     'hipmc_variance_update', 'hipmc_glm_hmc_run_noalloc',
@@ -135,6 +136,8 @@ def lib():
       l.hipmc_last_error.restype = ctypes.c_char_p
       for name in ('hipmc_hmc_run', 'hipmc_leapfrog_run', 'hipmc_nuts_run'):
         getattr(l, name).argtypes = [ctypes.POINTER(RunArgs), _u64]
+      l.hipmc_nuts_run_queued.argtypes = [ctypes.POINTER(RunArgs), _vp, _vp,
+                                          _u64]
       l.hipmc_glm_hmc_run.argtypes = [ctypes.POINTER(GlmHmcArgs), _u64]
       l.hipmc_glm_hmc_run_noalloc.argtypes = [ctypes.POINTER(GlmHmcArgs),
                                               _u64]
@@ -220,6 +223,7 @@ def stream_handle(device=None):
 
 
 MAX_COPY_BLOCKS = 16
+QUEUE_WORDS = 16
 
 
 def copy_blocks(blocks, elem_size, device, mask=None):

@@ -114,8 +114,9 @@ int by_family(int dtype, int kind, A&&... args) {
 
 template <typename T, int FAM>
 struct NutsL {
-  static int run(const hipmc_run_args& a, hipStream_t s) {
-    return launch_nuts_k<T, FAM>(pick_k(a.max_dim, FAM), a, s);
+  static int run(const hipmc_run_args& a, int32_t* queue,
+                 const int32_t* order, hipStream_t s) {
+    return launch_nuts_k<T, FAM>(pick_k(a.max_dim, FAM), a, queue, order, s);
   }
 };
 template <typename T, int FAM>
@@ -717,7 +718,16 @@ int hipmc_glm_hmc_run_noalloc(const hipmc_glm_hmc_args* a, uint64_t stream) {
 int hipmc_nuts_run(const hipmc_run_args* a, uint64_t stream) {
   int rc = check_run(a, true);
   if (rc) return rc;
-  return by_family<NutsL>(a->dtype, a->target_kind, *a, as_stream(stream));
+  return by_family<NutsL>(a->dtype, a->target_kind, *a, (int32_t*)nullptr,
+                          (const int32_t*)nullptr, as_stream(stream));
+}
+
+int hipmc_nuts_run_queued(const hipmc_run_args* a, int32_t* queue,
+                          const int32_t* order, uint64_t stream) {
+  int rc = check_run(a, true);
+  if (rc) return rc;
+  return by_family<NutsL>(a->dtype, a->target_kind, *a, queue, order,
+                          as_stream(stream));
 }
 
 int hipmc_hmc_run(const hipmc_run_args* a, uint64_t stream) {

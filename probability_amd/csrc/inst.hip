@@ -13,7 +13,7 @@
 namespace hipmc {
 #if HIPMC_INST_NUTS
 template int launch_nuts_k<HIPMC_INST_T, HIPMC_INST_FAM>(
-    int, const hipmc_run_args&, hipStream_t);
+    int, const hipmc_run_args&, int32_t*, const int32_t*, hipStream_t);
 #else
 template int launch_hmc_k<HIPMC_INST_T, HIPMC_INST_FAM>(
     int, bool, const hipmc_run_args&, hipStream_t);

@@ -619,6 +619,52 @@ __device__ __attribute__((always_inline)) inline void nuts_chain(
   if (lane == 0) ((T*)a.tlp)[crow] = (T)t0;
 }
 
+// Chains handed to the blocks that are ready for one (hipmc_nuts_run_queued):
+// word x of the queue counts the chains taken of list x, which XCD x's blocks
+// start from (the chains of a problem read the same data); a block whose list
+// is used up goes on with the next XCD's.  The last block to leave sets the
+// words back to zero for the next launch.  A trajectory's length is not known
+// before it is run, so any deal of whole chains to the XCDs (blocks go to them
+// in turn) leaves some of them idle at the end.  24 regressions of 173..7038
+// rows and 12..122 columns, 32 chains, 3 draws, whose chains take 2.97 ms of
+// every CU: 4.7 ms as dealt, 4.2 ms from the queue in the order of the
+// problems, 3.96 ms with each problem on one list and the costliest first (4.2
+// ms with its chains on all lists: its data then are on every XCD's L2).
+struct ChainQueue {
+  int step = 0;  // lists used up (thread 0)
+
+  // The block's next chain, or -1; `slot` is LDS that no wave holds data in.
+  // order: nine starts of the lists, then the chains; NULL: eighths of 0, 1..
+  __device__ int next(int32_t* queue, const int32_t* order, int n, int* slot) {
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      int c = -1;
+      for (; step < 8; ++step) {
+        const int x = (blockIdx.x + step) & 7;
+        const int per = n >> 3, rem = n & 7;
+        const int at = order ? order[x] : x * per + (x < rem ? x : rem);
+        const int len = order ? order[x + 1] - at : per + (x < rem ? 1 : 0);
+        const int i = atomicAdd(&queue[x], 1);
+        if (i < len) {
+          c = order ? order[9 + at + i] : at + i;
+          break;
+        }
+      }
+      *slot = c;
+    }
+    __syncthreads();
+    const int c = __builtin_amdgcn_readfirstlane(*slot);
+    __syncthreads();
+    return c;
+  }
+
+  __device__ void leave(int32_t* queue) {
+    if (threadIdx.x == 0 &&
+        atomicAdd(&queue[8], 1) == (int)gridDim.x - 1)
+      for (int x = 0; x < 9; ++x) queue[x] = 0;
+  }
+};
+
 // GLM chains are bound by loads in flight, so their kernel is built for two
 // waves per SIMD (the register budget that allows) and blocks of up to
 // eight waves (one chain shared by a whole CU); the other families keep one
@@ -626,7 +672,7 @@ __device__ __attribute__((always_inline)) inline void nuts_chain(
 template <typename T, int K, int FAM>
 __global__ void __launch_bounds__(FAM == kFamilyGlm ? 512 : 256)
     __attribute__((amdgpu_waves_per_eu(FAM == kFamilyGlm ? 2 : 1)))
-    nuts_kernel(hipmc_run_args a) {
+    nuts_kernel(hipmc_run_args a, int32_t* queue, const int32_t* order) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
   const int wave = threadIdx.x >> 6;
   const int waves = blockDim.x >> 6;
@@ -635,39 +681,52 @@ __global__ void __launch_bounds__(FAM == kFamilyGlm ? 512 : 256)
   // share of the rows, the partial sums meet in LDS, every wave runs the
   // same control flow on the same values); otherwise a wave per chain.
   const int W = waves_per_chain<FAM>(a);
-  const int c = W > 1 ? xcd_block(blockIdx.x, gridDim.x)
-                      : xcd_block(blockIdx.x, gridDim.x) * waves + wave;
+  const bool queued = FAM == kFamilyGlm && W > 1 && queue != nullptr;
+  ChainQueue cq;
+  int c = xcd_block(blockIdx.x, gridDim.x);
+  if (W == 1) c = c * waves + wave;
+  if (queued) c = cq.next(queue, order, a.n_chains, (int*)smem_raw);
   const int wic = W > 1 ? wave : 0;
-  if (c >= a.n_chains) return;  // whole wave (block, if shared) leaves
-  const size_t cl = nuts_chain_lds_elems<T, K, FAM>(max_depth);
-  const size_t wl = nuts_wave_lds_elems<T, K, FAM>();
-  const size_t scr = target_scratch_elems<T, K, FAM>();
-  // W > 1: [chain block][W wave blocks][partial-sum halves];
-  // W == 1: one [chain block, wave block] per wave
-  T* chain_base = W > 1 ? (T*)smem_raw : (T*)smem_raw + (size_t)wave * (cl + wl);
-  T* wave_base = W > 1 ? (T*)smem_raw + cl + (size_t)wic * wl : chain_base + cl;
-  T* memP = chain_base;  // one copy per chain; the waves of a chain write equal values
-  T* memC = chain_base + (size_t)max_depth * K * 64;
-  T* tree = chain_base + (size_t)2 * max_depth * K * 64;
-  T* scratch = wave_base;
-  T* leafp = wave_base + scr;
+  // the whole wave (block, if shared) leaves
+  while (c >= 0 && c < a.n_chains) {
+    const size_t cl = nuts_chain_lds_elems<T, K, FAM>(max_depth);
+    const size_t wl = nuts_wave_lds_elems<T, K, FAM>();
+    const size_t scr = target_scratch_elems<T, K, FAM>();
+    // W > 1: [chain block][W wave blocks][partial-sum halves];
+    // W == 1: one [chain block, wave block] per wave
+    T* chain_base =
+        W > 1 ? (T*)smem_raw : (T*)smem_raw + (size_t)wave * (cl + wl);
+    T* wave_base =
+        W > 1 ? (T*)smem_raw + cl + (size_t)wic * wl : chain_base + cl;
+    // one copy per chain; the waves of a chain write equal values
+    T* memP = chain_base;
+    T* memC = chain_base + (size_t)max_depth * K * 64;
+    T* tree = chain_base + (size_t)2 * max_depth * K * 64;
+    T* scratch = wave_base;
+    T* leafp = wave_base + scr;
 
-  const ChainId id = chain_of(a, c);
-  const hipmc_problem& pb = a.problems[id.prob];
-  Target<T, K, FAM> tg;
-  tg.load(pb, scratch);
-  if (W > 1) tg.set_split(wic, W, (unsigned char*)((T*)smem_raw + cl + (size_t)W * wl));
-  const bool u1 = a.unrolled_leapfrog_steps == 1;
-  if (FAM == kFamilyHier && u1 && tg.sp0) {
-    nuts_chain<T, K, FAM, kBijSlot0Softplus, true>(a, tg, id, c, wic, W, memP,
-                                                    memC, tree, leafp, pb);
-  } else if (u1) {
-    nuts_chain<T, K, FAM, kBijAny, true>(a, tg, id, c, wic, W, memP, memC,
-                                         tree, leafp, pb);
-  } else {
-    nuts_chain<T, K, FAM, kBijAny, false>(a, tg, id, c, wic, W, memP, memC,
-                                          tree, leafp, pb);
+    const ChainId id = chain_of(a, c);
+    const hipmc_problem& pb = a.problems[id.prob];
+    Target<T, K, FAM> tg;
+    tg.load(pb, scratch);
+    if (W > 1)
+      tg.set_split(wic, W,
+                   (unsigned char*)((T*)smem_raw + cl + (size_t)W * wl));
+    const bool u1 = a.unrolled_leapfrog_steps == 1;
+    if (FAM == kFamilyHier && u1 && tg.sp0) {
+      nuts_chain<T, K, FAM, kBijSlot0Softplus, true>(
+          a, tg, id, c, wic, W, memP, memC, tree, leafp, pb);
+    } else if (u1) {
+      nuts_chain<T, K, FAM, kBijAny, true>(a, tg, id, c, wic, W, memP, memC,
+                                           tree, leafp, pb);
+    } else {
+      nuts_chain<T, K, FAM, kBijAny, false>(a, tg, id, c, wic, W, memP, memC,
+                                            tree, leafp, pb);
+    }
+    if (!queued) return;
+    c = cq.next(queue, order, a.n_chains, (int*)smem_raw);
   }
+  if (queued) cq.leave(queue);
 }
 
 // Chain groups (GLM): G chains of one problem per block, chain j's NUTS run

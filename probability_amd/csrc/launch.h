@@ -20,6 +20,17 @@ int allow_lds(F* kernel, size_t bytes) {
                    "hipFuncSetAttribute(max dynamic LDS)");
 }
 
+// CUs of the current device.
+inline int device_cus() {
+  int dev = 0, n = 0;
+  if (hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) !=
+          hipSuccess ||
+      n < 1)
+    return 256;
+  return n;
+}
+
 inline int waves_for_lds(size_t per_wave_bytes) {
   int w = 4;
   while (w > 1 && (size_t)w * per_wave_bytes > (size_t)kMaxLdsPerBlock) --w;
@@ -65,7 +76,8 @@ int try_launch_nuts_group(const hipmc_run_args& a, hipStream_t s) {
 }
 
 template <typename T, int K, int FAM>
-int launch_nuts(const hipmc_run_args& a0, hipStream_t s) {
+int launch_nuts(const hipmc_run_args& a0, int32_t* queue,
+                const int32_t* order, hipStream_t s) {
   if (a0.n_chains == 0) return HIPMC_OK;
   {
     const int rc = try_launch_nuts_group<T, K, FAM>(a0, s);
@@ -88,8 +100,13 @@ int launch_nuts(const hipmc_run_args& a0, hipStream_t s) {
     const size_t bytes = shared_bytes(W);
     const int rc = allow_lds(&nuts_kernel<T, K, FAM>, bytes);
     if (rc != HIPMC_OK) return rc;
-    hipLaunchKernelGGL((nuts_kernel<T, K, FAM>), dim3(a.n_chains),
-                       dim3(64 * W), bytes, s, a);
+    // blocks of 8 waves share a chain at two waves per SIMD, so 8 / W blocks
+    // fit a CU; more chains than that are handed out as blocks get ready
+    const int resident = device_cus() * (8 / W);
+    if (a.n_chains <= resident) queue = nullptr;
+    hipLaunchKernelGGL((nuts_kernel<T, K, FAM>),
+                       dim3(queue ? resident : a.n_chains), dim3(64 * W),
+                       bytes, s, a, queue, order);
     return hip_check(hipGetLastError(), "nuts_kernel launch");
   }
   const size_t per_wave = (cl + wl) * sizeof(T);
@@ -103,13 +120,13 @@ int launch_nuts(const hipmc_run_args& a0, hipStream_t s) {
     const int rc = allow_lds(&nuts_kernel<T, K, FAM>, per_wave);
     if (rc != HIPMC_OK) return rc;
     hipLaunchKernelGGL((nuts_kernel<T, K, FAM>), dim3(a.n_chains), dim3(64),
-                       per_wave, s, a);
+                       per_wave, s, a, (int32_t*)nullptr, (const int32_t*)nullptr);
     return hip_check(hipGetLastError(), "nuts_kernel launch");
   }
   const int w = waves_for_lds(per_wave);
   const int blocks = (a.n_chains + w - 1) / w;
   hipLaunchKernelGGL((nuts_kernel<T, K, FAM>), dim3(blocks), dim3(64 * w),
-                     per_wave * w, s, a);
+                     per_wave * w, s, a, (int32_t*)nullptr, (const int32_t*)nullptr);
   return hip_check(hipGetLastError(), "nuts_kernel launch");
 }
 
@@ -165,10 +182,11 @@ static_assert(max_slots(kFamilyGlm) == 8 && max_slots(kFamilyHier) == 17 &&
               "slot lists and max_slots disagree");
 
 template <typename T, int FAM>
-int launch_nuts_k(int k, const hipmc_run_args& a, hipStream_t s) {
+int launch_nuts_k(int k, const hipmc_run_args& a, int32_t* queue,
+                  const int32_t* order, hipStream_t s) {
   switch (k) {
 #define HIPMC_CASE(KK) \
-  case KK: return launch_nuts<T, KK, FAM>(a, s);
+  case KK: return launch_nuts<T, KK, FAM>(a, queue, order, s);
     HIPMC_FOR_EACH_K(HIPMC_CASE)
   }
   if constexpr (FAM != kFamilyGlm) {

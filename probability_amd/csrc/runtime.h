@@ -40,7 +40,8 @@ int max_state_dim(int fam);
 // Sampling-kernel launchers of one (dtype T, family FAM) pair; k is the
 // register slot count from pick_k.
 template <typename T, int FAM>
-int launch_nuts_k(int k, const hipmc_run_args& a, hipStream_t s);
+int launch_nuts_k(int k, const hipmc_run_args& a, int32_t* queue,
+                  const int32_t* order, hipStream_t s);
 template <typename T, int FAM>
 int launch_hmc_k(int k, bool calibrated, const hipmc_run_args& a,
                  hipStream_t s);

@@ -113,6 +113,7 @@ class PosteriorBatch:
     if _family(self.kind) == 2 and len({s.kind for s in self.specs}) > 1:
       self.kind = _lib.TARGET_DIAG_NORMAL
     self._tiles = None  # of eval()
+    self._order = None  # of start_order()
     if fams == {1}:
       cols = max(d - (s.kind == _lib.TARGET_LINEAR)
                  for s, d in zip(self.specs, self.dims))
@@ -139,6 +140,17 @@ class PosteriorBatch:
   @property
   def n_problems(self):
     return len(self.specs)
+
+  def start_order(self):
+    """Device array: the order in which the chains of a NUTS launch start
+    (hipmc_nuts_run_queued), or None where it does not matter."""
+    if self._order is None:
+      cost = ([_leaf_cost(s, self.dtype) for s in self.specs]
+              if _family(self.kind) == 1 and self.waves_per_chain > 1 else [0])
+      self._order = (torch.as_tensor(
+          _start_order(cost, self.num_chains), device=self.device)
+                     if min(cost) < max(cost) else None,)
+    return self._order[0]
 
   def eval(self, x):
     """(tlp [C], grad [C, dim_stride]) of every chain at x."""
@@ -183,6 +195,30 @@ class PosteriorBatch:
     """Per-problem views [..., C_p] of a [..., C] array."""
     return [arr[..., int(self.chain_offsets[i]):int(self.chain_offsets[i + 1])]
             for i in range(self.n_problems)]
+
+
+def _leaf_cost(spec, dtype):
+  """Microseconds of one leapfrog of a GLM chain on a CU of its own (eight
+  waves): 7 for the trajectory's bookkeeping, and per 1000 rows 0.3 and 2.1
+  for every block of coefficients (measured 6.9 at 192 x 31, 9.4 at 1443 x 42,
+  23.5 at 7038 x 34, 17.9 at 2842 x 118, 27.2 at 4359 x 86 with 64 elements to
+  the block)."""
+  block = 64 if dtype == torch.float32 else 32
+  return 7.0 + spec.n_obs * (3e-4 + 2.1e-3 * -(-spec.dim // block))
+
+
+def _start_order(cost, num_chains, n_xcd=8):
+  """Order of hipmc_nuts_run_queued: the problems, those with the costliest
+  leapfrogs first, dealt to the XCDs' lists in snake order."""
+  ends = np.cumsum(num_chains)
+  lists = [[] for _ in range(n_xcd)]
+  for r, i in enumerate(np.argsort(-np.asarray(cost), kind='stable')):
+    k = r % (2 * n_xcd)
+    lists[k if k < n_xcd else 2 * n_xcd - 1 - k].append(
+        np.arange(ends[i] - num_chains[i], ends[i]))
+  sizes = [sum(map(len, c)) for c in lists]
+  return np.concatenate(
+      [[0], np.cumsum(sizes)] + sum(lists, [])).astype(np.int32)
 
 
 def sample_posteriors(batch, num_results, num_burnin_steps=0,
@@ -505,6 +541,10 @@ class _Run:
       self.div = torch.zeros((rows, c), dtype=torch.uint8, device=dev)
       self.tr = (torch.empty((num_results, c, d), dtype=dt, device=dev)
                  if trace else None)
+      # of this run's NUTS launches, one at a time on its stream
+      self.queue = torch.zeros(_lib.QUEUE_WORDS, dtype=torch.int32,
+                               device=dev)
+      self.order = batch.start_order() if kernel == 'nuts' else None
       # windowed adaptation: diagonal momentum precision per problem, the
       # running variance it is estimated from, and the window bookkeeping
       self.prec = None
@@ -524,8 +564,6 @@ class _Run:
         self.corr = torch.empty((max(self.n_total, 1), c), dtype=dt,
                                 device=dev)
     self.base_seed = samplers.sanitize_seed(seed, salt='mcmc.sample_chain')
-    self.fn = (_lib.lib().hipmc_nuts_run if kernel == 'nuts'
-               else _lib.lib().hipmc_hmc_run)
     self.events = ([] if (stats is not None and stats.get('time_kernels'))
                    else None)
     self.t = 0
@@ -664,7 +702,14 @@ class _Run:
       e0 = torch.cuda.Event(enable_timing=True)
       e1 = torch.cuda.Event(enable_timing=True)
       e0.record()
-    _lib.check(self.fn(a, _lib.stream_handle(b.device)))
+    if self.kernel == 'nuts':
+      rc = _lib.lib().hipmc_nuts_run_queued(
+          a, self.queue.data_ptr(),
+          None if self.order is None else self.order.data_ptr(),
+          _lib.stream_handle(b.device))
+    else:
+      rc = _lib.lib().hipmc_hmc_run(a, _lib.stream_handle(b.device))
+    _lib.check(rc)
     if self.events is not None:
       e1.record()
       self.events.append((e0, e1, t0, n))
