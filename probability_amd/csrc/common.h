@@ -308,58 +308,71 @@ __device__ inline A row_sum_pick4(A a0, A a1, A a2, A a3, bool b0, bool b1) {
 __device__ inline float wave_sum(float v) { return rows_total(row_sum(v)); }
 __device__ inline double wave_sum(double v) { return rows_total(row_sum(v)); }
 
-// Two independent sums reduced together (interleaved for latency).
-template <typename A, typename B>
-__device__ inline void wave_sum2(A a, B b, A& ra, B& rb) {
-  a = dpp_add<kDppQuadXor1>(a);
-  b = dpp_add<kDppQuadXor1>(b);
-  a = dpp_add<kDppQuadXor2>(a);
-  b = dpp_add<kDppQuadXor2>(b);
-  a = dpp_add<kDppHalfMirror>(a);
-  b = dpp_add<kDppHalfMirror>(b);
-  a = dpp_add<kDppMirror>(a);
-  b = dpp_add<kDppMirror>(b);
-  a = dpp_add_rows<kDppRowBcast15, 0xA>(a);
-  b = dpp_add_rows<kDppRowBcast15, 0xA>(b);
-  a = dpp_add_rows<kDppRowBcast31, 0xC>(a);
-  b = dpp_add_rows<kDppRowBcast31, 0xC>(b);
-  ra = readlane(a, 63);
-  rb = readlane(b, 63);
+// (r0 + r1) + (r2 + r3) of the row sums r0..r3 of each lane column, in every
+// row (rows_total's adds, which are commutative): a permlane swap of two
+// copies leaves a row's own sum and its partner's side by side.
+__device__ inline float rows_add(float v) {
+  const uint32_t u = __float_as_uint(v);
+  const auto p = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+  const uint32_t w = __float_as_uint(__uint_as_float(p[0]) +
+                                     __uint_as_float(p[1]));
+  const auto q = __builtin_amdgcn_permlane32_swap(w, w, false, false);
+  return __uint_as_float(q[0]) + __uint_as_float(q[1]);
+}
+__device__ inline double rows_add(double v) {
+  auto both = [](double x, auto swap) {
+    const uint64_t b = (uint64_t)__double_as_longlong(x);
+    const auto lo = swap((uint32_t)b), hi = swap((uint32_t)(b >> 32));
+    return __longlong_as_double((int64_t)(((uint64_t)hi[0] << 32) | lo[0])) +
+           __longlong_as_double((int64_t)(((uint64_t)hi[1] << 32) | lo[1]));
+  };
+  v = both(v, [](uint32_t u) {
+    return __builtin_amdgcn_permlane16_swap(u, u, false, false);
+  });
+  return both(v, [](uint32_t u) {
+    return __builtin_amdgcn_permlane32_swap(u, u, false, false);
+  });
 }
 
-// Four independent wave sums with their DPP stages interleaved (each sum
-// in the order of wave_sum).
+// Two independent sums reduced together, each in the order of wave_sum: once
+// every lane of a quad holds its quad's sums, lanes 0 and 3 of the quad go on
+// with the first and lanes 1 and 2 with the second (the mirrors keep them
+// apart), in 15 instructions for floats (22 as two sums) and 34 for doubles
+// (50).
 template <typename A>
-__device__ inline void wave_sum4(A a, A b, A c, A d, A& ra, A& rb, A& rc,
-                                 A& rd) {
+__device__ inline void wave_sum2(A a, A b, A& ra, A& rb) {
+  const int lane = lane_id();
   a = dpp_add<kDppQuadXor1>(a);
   b = dpp_add<kDppQuadXor1>(b);
-  c = dpp_add<kDppQuadXor1>(c);
-  d = dpp_add<kDppQuadXor1>(d);
   a = dpp_add<kDppQuadXor2>(a);
   b = dpp_add<kDppQuadXor2>(b);
-  c = dpp_add<kDppQuadXor2>(c);
-  d = dpp_add<kDppQuadXor2>(d);
-  a = dpp_add<kDppHalfMirror>(a);
-  b = dpp_add<kDppHalfMirror>(b);
-  c = dpp_add<kDppHalfMirror>(c);
-  d = dpp_add<kDppHalfMirror>(d);
-  a = dpp_add<kDppMirror>(a);
-  b = dpp_add<kDppMirror>(b);
-  c = dpp_add<kDppMirror>(c);
-  d = dpp_add<kDppMirror>(d);
-  a = dpp_add_rows<kDppRowBcast15, 0xA>(a);
-  b = dpp_add_rows<kDppRowBcast15, 0xA>(b);
-  c = dpp_add_rows<kDppRowBcast15, 0xA>(c);
-  d = dpp_add_rows<kDppRowBcast15, 0xA>(d);
-  a = dpp_add_rows<kDppRowBcast31, 0xC>(a);
-  b = dpp_add_rows<kDppRowBcast31, 0xC>(b);
-  c = dpp_add_rows<kDppRowBcast31, 0xC>(c);
-  d = dpp_add_rows<kDppRowBcast31, 0xC>(d);
-  ra = readlane(a, 63);
-  rb = readlane(b, 63);
-  rc = readlane(c, 63);
-  rd = readlane(d, 63);
+  A v = ((lane ^ (lane >> 1)) & 1) ? b : a;
+  v = dpp_add<kDppHalfMirror>(v);
+  v = rows_add(dpp_add<kDppMirror>(v));
+  ra = readlane(v, 0);
+  rb = readlane(v, 1);
+}
+
+// Whether the sums of a and b, and of c and d (wave_sum each), are at least
+// zero; false for NaN.  The sums stay in the lanes: no lane is read.
+template <typename A>
+__device__ inline bool sums_nonneg(A a, A b, A c, A d) {
+  const int lane = lane_id();
+  const A v = rows_add(
+      row_sum_pick4(a, b, c, d, (lane & 1) != 0, (lane & 2) != 0));
+  return __ballot(!(v >= A(0))) == 0;
+}
+template <typename A>
+__device__ inline bool sums_nonneg(A a, A b) {
+  const int lane = lane_id();
+  a = dpp_add<kDppQuadXor1>(a);
+  b = dpp_add<kDppQuadXor1>(b);
+  a = dpp_add<kDppQuadXor2>(a);
+  b = dpp_add<kDppQuadXor2>(b);
+  A v = ((lane ^ (lane >> 1)) & 1) ? b : a;
+  v = dpp_add<kDppHalfMirror>(v);
+  v = rows_add(dpp_add<kDppMirror>(v));
+  return __ballot(!(v >= A(0))) == 0;
 }
 
 // ---------------------------------------------------------------- scalars

@@ -345,7 +345,10 @@ __host__ __device__ constexpr size_t nuts_lds_elems(int max_depth) {
 // W > 1: the W waves of one block share the chain (GLMs); they run the same
 // control flow on identical values, and their parked tree vectors are one
 // copy guarded by a block barrier before each write.
-template <typename T, int K, int FAM, int BM, bool U1, int G = 1>
+// PRE = false: no momentum precision, whatever the launch's; only where the
+// caller has checked that there is none.
+template <typename T, int K, int FAM, int BM, bool U1, int G = 1,
+          bool PRE = true>
 __device__ __attribute__((always_inline)) inline void nuts_chain(
     const hipmc_run_args& a, Target<T, K, FAM, G>& tg, const ChainId& id,
     int c, int wic, int W, T* memP, T* memC, T* tree, T* leafp,
@@ -362,7 +365,14 @@ __device__ __attribute__((always_inline)) inline void nuts_chain(
 
   T m[K];
   double kconst;
-  const bool pre = load_precision(a, id, dim, m, kconst);
+  bool pre = false;
+  if (PRE) {
+    pre = load_precision(a, id, dim, m, kconst);
+  } else {
+    kconst = 0.0;
+#pragma unroll
+    for (int k = 0; k < K; ++k) m[k] = T(1);
+  }
   T q0[K], g0[K];
   load_row(q0, (const T*)a.state + row, dim);
   load_row(g0, (const T*)a.grad + row, dim);
@@ -430,8 +440,7 @@ __device__ __attribute__((always_inline)) inline void nuts_chain(
       // Per-lane buffers for 64 consecutive leaves: lane l holds leaf
       // (chunk + l)'s log1p(-U) (drawn for the whole chunk at once) and its
       // energy difference, whose exp(min(dH, 0)) terms are summed per chunk.
-      double lu_buf = 0.0, de_buf = 0.0;
-      bool de_ok = false;
+      double lu_buf = 0.0, de_buf = neg_inf();
       for (int i = 0; i < nsteps; ++i) {
         // _loop_build_sub_tree (nuts.py:793-946)
         const int li = i & 63;
@@ -448,7 +457,7 @@ __device__ __attribute__((always_inline)) inline void nuts_chain(
 #pragma unroll
           for (int k = 0; k < K; ++k) {
             p[k] = p[k] + half * g[k];
-            q[k] = q[k] + e * (m[k] * p[k]);
+            q[k] = q[k] + e * (PRE ? m[k] * p[k] : p[k]);
           }
           if (PARK) {
             park(leafp + 0 * S, p); park(leafp + 1 * S, cs);
@@ -465,7 +474,7 @@ __device__ __attribute__((always_inline)) inline void nuts_chain(
           for (int k = 0; k < K; ++k) {
             p[k] = p[k] + e * g[k];
             p[k] = p[k] - half * g[k];
-            v[k] = m[k] * p[k];
+            v[k] = PRE ? m[k] * p[k] : p[k];
             kin += (double)p[k] * (double)v[k];
           }
           double slp, skin;
@@ -507,31 +516,36 @@ __device__ __attribute__((always_inline)) inline void nuts_chain(
           __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
           __builtin_amdgcn_wave_barrier();
           __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-          // Two checks per round, their reductions interleaved; the result
-          // is the AND of the same per-slot tests (a lone last check is
-          // evaluated twice).
+          // two checks per round, their four sums reduced together, and a
+          // last one by itself
           const int top = __popc(i);
-          const int lo = top - __builtin_ctz((unsigned)(i + 1));
-          for (int j = lo; j < top && no_u; j += 2) {
-            const int j1 = j + 1 < top ? j + 1 : j;
+          int j = top - __builtin_ctz((unsigned)(i + 1));
+          for (; j + 1 < top && no_u; j += 2) {
             const T* mp0 = memP + (size_t)j * K * 64;
             const T* mc0 = memC + (size_t)j * K * 64;
-            const T* mp1 = memP + (size_t)j1 * K * 64;
-            const T* mc1 = memC + (size_t)j1 * K * 64;
             T sl0 = T(0), sr0 = T(0), sl1 = T(0), sr1 = T(0);
 #pragma unroll
             for (int k = 0; k < K; ++k) {
               const T d0 = cs[k] - mc0[k * 64 + lane];
-              const T d1 = cs[k] - mc1[k * 64 + lane];
+              const T d1 = cs[k] - mc0[(K + k) * 64 + lane];
               sl0 += d0 * mp0[k * 64 + lane];
               sr0 += d0 * v[k];
-              sl1 += d1 * mp1[k * 64 + lane];
+              sl1 += d1 * mp0[(K + k) * 64 + lane];
               sr1 += d1 * v[k];
             }
-            T dl0, dr0, dl1, dr1;
-            wave_sum4(sl0, sr0, sl1, sr1, dl0, dr0, dl1, dr1);
-            no_u = (dl0 >= T(0)) && (dr0 >= T(0)) && (dl1 >= T(0)) &&
-                   (dr1 >= T(0));
+            no_u = sums_nonneg(sl0, sr0, sl1, sr1);
+          }
+          if (j < top && no_u) {
+            const T* mp0 = memP + (size_t)j * K * 64;
+            const T* mc0 = memC + (size_t)j * K * 64;
+            T sl0 = T(0), sr0 = T(0);
+#pragma unroll
+            for (int k = 0; k < K; ++k) {
+              const T d0 = cs[k] - mc0[k * 64 + lane];
+              sl0 += d0 * mp0[k * 64 + lane];
+              sr0 += d0 * v[k];
+            }
+            no_u = sums_nonneg(sl0, sr0);
           }
         }
         if (__builtin_isnan(energy)) energy = neg_inf();
@@ -547,13 +561,14 @@ __device__ __attribute__((always_inline)) inline void nuts_chain(
         }
         wS = wsum;
         // energy_diff_sum counts the steps that continue
-        de_buf = lane == li ? de : de_buf;
-        de_ok = lane == li ? not_div : de_ok;
+        const double de_in = not_div ? de : neg_inf();  // exp: no term
+        de_buf = lane == li ? de_in : de_buf;
         nd = nd && not_div;
         csub = not_div && no_u;
         if (li == 63 || !csub || i + 1 == nsteps) {
-          eds_sub += wave_sum(de_ok ? exp(fmin(de_buf, 0.0)) : 0.0);
-          de_ok = false;
+          keep_branch();
+          eds_sub += wave_sum(exp(fmin(de_buf, 0.0)));
+          de_buf = neg_inf();
         }
         if (!csub) break;
       }
@@ -665,6 +680,14 @@ struct ChainQueue {
   }
 };
 
+// Between its gradients a leaf is bound by the instructions its wave issues,
+// four cycles each and one after the other (in every wave of a shared chain):
+// with scalar branches, the leaf's sums reduced in pairs and fours that share
+// their last stages, a lone U-turn check not doubled, and no masks, precisions
+// or products by one where there are none (kBijSlot0SoftplusFull), a leaf of
+// 258 elements takes 195 vector instructions and 1390 cycles (236 and 1560;
+// the time of 1024 such chains fell by 0 to 5%, as the clock did not hold).
+// 24 ragged regressions x 32 chains, 3 draws: 4.34 -> 3.79 ms.
 // GLM chains are bound by loads in flight, so their kernel is built for two
 // waves per SIMD (the register budget that allows) and blocks of up to
 // eight waves (one chain shared by a whole CU); the other families keep one
@@ -674,7 +697,9 @@ __global__ void __launch_bounds__(FAM == kFamilyGlm ? 512 : 256)
     __attribute__((amdgpu_waves_per_eu(FAM == kFamilyGlm ? 2 : 1)))
     nuts_kernel(hipmc_run_args a, int32_t* queue, const int32_t* order) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
-  const int wave = threadIdx.x >> 6;
+  // a scalar: what hangs on the chain (its pointers, step, log-prob and with
+  // them the trajectory's branches) is then scalar too, not exec masks
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int waves = blockDim.x >> 6;
   const int max_depth = a.max_tree_depth;
   // GLM chains may be shared by the W waves of a block (each evaluates a
@@ -713,7 +738,15 @@ __global__ void __launch_bounds__(FAM == kFamilyGlm ? 512 : 256)
       tg.set_split(wic, W,
                    (unsigned char*)((T*)smem_raw + cl + (size_t)W * wl));
     const bool u1 = a.unrolled_leapfrog_steps == 1;
-    if (FAM == kFamilyHier && u1 && tg.sp0) {
+    // float only: there the products that the masks and precisions keep apart
+    // from the sums are exact in the sums' double, so the results are the same
+    constexpr bool kFull = FAM == kFamilyHier && K <= 5 && sizeof(T) == 4;
+    if (kFull && u1 && tg.sp0 && pb.dim > 64 * (K - 1) &&
+        !a.momentum_precision) {
+      nuts_chain<T, K, FAM, kFull ? kBijSlot0SoftplusFull : kBijSlot0Softplus,
+                 true, 1, !kFull>(a, tg, id, c, wic, W, memP, memC, tree,
+                                  leafp, pb);
+    } else if (FAM == kFamilyHier && u1 && tg.sp0) {
       nuts_chain<T, K, FAM, kBijSlot0Softplus, true>(
           a, tg, id, c, wic, W, memP, memC, tree, leafp, pb);
     } else if (u1) {
@@ -750,7 +783,7 @@ template <typename T, int K, int G>
 __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2)))
     nuts_group_kernel(hipmc_run_args a) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
-  const int wave = threadIdx.x >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int W = blockDim.x >> 6;
   const int max_depth = a.max_tree_depth;
   const int c0 = xcd_block(blockIdx.x, gridDim.x) * G;
@@ -794,7 +827,7 @@ template <typename T, int K, int FAM, bool CALIBRATED>
 __global__ void __launch_bounds__(256) hmc_kernel(hipmc_run_args a) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
   const int lane = lane_id();
-  const int wave = threadIdx.x >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int waves = blockDim.x >> 6;
   // GLM chains may be shared by the W waves of a block (as in nuts_kernel)
   const int W = waves_per_chain<FAM>(a);
@@ -898,7 +931,7 @@ __global__ void __launch_bounds__(256)
                 int n_chains, int dim_stride, const T* x, T* out_tlp,
                 T* out_grad) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
-  const int wave = threadIdx.x >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int waves = blockDim.x >> 6;
   const int c = blockIdx.x * waves + wave;
   if (c >= n_chains) return;

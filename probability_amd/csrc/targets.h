@@ -119,6 +119,8 @@ __device__ inline void put_slot(T (&v)[K], int s, T f) {
 // Bijector code paths of Target::eval_partial.
 constexpr int kBijAny = 0;            // chosen at run time from the layout
 constexpr int kBijSlot0Softplus = 1;  // every bijector lane: Softplus, slot 0
+// the same, and every slot but the last is full of state elements
+constexpr int kBijSlot0SoftplusFull = 2;
 
 // Shared LDS of a chain group (G chains of one GLM problem whose owner
 // waves take turns with all W waves of the block streaming X once for every
@@ -276,7 +278,8 @@ struct Target : RowSums<T, K, G> {
   // the gradient.  The caller reduces the partial (possibly together with
   // other sums).  Bijector log-det-Jacobians are folded into the partial.
   // BM = kBijSlot0Softplus compiles only the path for bijectors that are all
-  // Softplus in register slot 0 (the caller has checked sp0); kBijAny
+  // Softplus in register slot 0 (the caller has checked sp0), and its Full
+  // form leaves out the masks of slots that hold state only; kBijAny
   // chooses the path at run time.
   template <int BM = kBijAny>
   __device__ double eval_partial(const T (&xs)[K], T (&g)[K], double& lpu) {
@@ -289,11 +292,11 @@ struct Target : RowSums<T, K, G> {
     // branches); otherwise the per-slot loop
     SoftplusParts<T> spb{};
     T exb = T(0);
-    if (BM == kBijSlot0Softplus || sp0) {
+    if (BM != kBijAny || sp0) {
       spb = softplus_parts(xs[0]);
       th[0] = code[0] == HIPMC_BIJ_SOFTPLUS ? fmax(xs[0], T(0)) + spb.l
                                             : xs[0];
-    } else if (BM == kBijSlot0Softplus) {
+    } else if (BM != kBijAny) {
     } else if (one_slot) {
       const T xb = pick(xs, bslot);
       if (sp_slots) spb = softplus_parts(xb);
@@ -323,7 +326,7 @@ struct Target : RowSums<T, K, G> {
     }
     double lpl;
     if (FAM == kFamilyHier) {
-      lpl = hier_normal(th, g, lpu);
+      lpl = hier_normal<BM == kBijSlot0SoftplusFull>(th, g, lpu);
     } else if (FAM == kFamilyGlm) {
       lpl = kind == HIPMC_TARGET_LINEAR ? glm<true>(th, g, lpu)
                                         : glm<false>(th, g, lpu);
@@ -337,11 +340,11 @@ struct Target : RowSums<T, K, G> {
     }
     // fldj: Softplus -softplus(-x) with d/dx f = sigmoid(x),
     // d/dx fldj = sigmoid(-x); Exp x with d/dx f = exp(x), d/dx fldj = 1
-    if (BM == kBijSlot0Softplus || sp0) {
+    if (BM != kBijAny || sp0) {
       const bool on = code[0] == HIPMC_BIJ_SOFTPLUS;
       lpl += on ? (double)(-(fmax(-xs[0], T(0)) + spb.l)) : 0.0;
       g[0] = on ? g[0] * spb.sig + spb.sig_neg : g[0];
-    } else if (BM == kBijSlot0Softplus) {
+    } else if (BM != kBijAny) {
     } else if (one_slot) {
       const T xb = pick(xs, bslot);
       const T gb = pick(g, bslot);
@@ -382,6 +385,8 @@ struct Target : RowSums<T, K, G> {
 
   // [mu, tau, z_0..z_{J-1}], y ~ N(mu + tau z, sigma); mu ~ N(0, p0),
   // tau ~ HalfCauchy(0, p1), z ~ N(0, 1).
+  // FULL: dim > 64 (K - 1), so slots 1..K-2 hold z's only.
+  template <bool FULL>
   __device__ double hier_normal(const T (&th)[K], T (&g)[K], double& lpu) {
     const int lane = lane_id();
     const T mu = readlane(th[0], 0);
@@ -391,15 +396,19 @@ struct Target : RowSums<T, K, G> {
 #pragma unroll
     for (int k = 0; k < K; ++k) {
       const int e = k * 64 + lane;
-      const bool is_z = (e >= 2) && (e < dim);
+      const bool is_z = (FULL && k > 0 && k < K - 1) ||
+                        ((e >= 2) && (e < dim));
       const T z = th[k];
       const T t = mu + tau * z;
       const T u = (a[k] - t) * b[k];  // (y - theta) / sigma
       const T r = u * b[k];           // (y - theta) / sigma^2
+      T rs = is_z ? r : T(0), rz = is_z ? r * z : T(0);
+      // without their masks the products would be fused into the sums
+      if (FULL) asm("" : "+v"(rs), "+v"(rz));
       lpl += is_z ? (double)(T(-0.5) * z * z - T(0.5) * u * u) : 0.0;
       g[k] = is_z ? (-z + tau * r) : T(0);
-      s1 += is_z ? r : T(0);
-      s2 += is_z ? r * z : T(0);
+      s1 += rs;
+      s2 += rz;
     }
     T S1, S2;
     wave_sum2(s1, s2, S1, S2);
