@@ -681,13 +681,13 @@ struct ChainQueue {
 };
 
 // Between its gradients a leaf is bound by the instructions its wave issues,
-// four cycles each and one after the other (in every wave of a shared chain):
-// with scalar branches, the leaf's sums reduced in pairs and fours that share
-// their last stages, a lone U-turn check not doubled, and no masks, precisions
-// or products by one where there are none (kBijSlot0SoftplusFull), a leaf of
-// 258 elements takes 195 vector instructions and 1390 cycles (236 and 1560;
-// the time of 1024 such chains fell by 0 to 5%, as the clock did not hold).
-// 24 ragged regressions x 32 chains, 3 draws: 4.34 -> 3.79 ms.
+// four cycles each and one after the other (in every wave of a shared chain).
+// The leaf's sums are reduced in pairs and fours that share their last stages,
+// a lone U-turn check is not doubled, and there are no masks, precisions or
+// products by one where there is nothing to mask (kBijSlot0SoftplusFull): 236
+// -> 195 vector instructions for 258 elements.  20 transitions of 256 groups,
+// 1024 chains (longest 1023 leaves) 8.15 -> 7.03 ms; 24 ragged regressions x 32
+// chains, 3 draws 4.34 -> 3.79 ms.
 // GLM chains are bound by loads in flight, so their kernel is built for two
 // waves per SIMD (the register budget that allows) and blocks of up to
 // eight waves (one chain shared by a whole CU); the other families keep one
@@ -697,9 +697,14 @@ __global__ void __launch_bounds__(FAM == kFamilyGlm ? 512 : 256)
     __attribute__((amdgpu_waves_per_eu(FAM == kFamilyGlm ? 2 : 1)))
     nuts_kernel(hipmc_run_args a, int32_t* queue, const int32_t* order) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
-  // a scalar: what hangs on the chain (its pointers, step, log-prob and with
-  // them the trajectory's branches) is then scalar too, not exec masks
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  // GLMs: a scalar, so that what hangs on the chain (its pointers, step,
+  // log-prob and with them the trajectory's branches) is scalar too: 24 ragged
+  // regressions x 32 chains, 3 draws 3.79 ms, with exec masks 4.35.  The other
+  // families' leaf, one wave per SIMD, is faster under exec masks than through
+  // branches: 20 transitions of 256 groups, 1024 chains 7.03 ms, scalar 8.17.
+  const int wave = FAM == kFamilyGlm
+                       ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6)
+                       : threadIdx.x >> 6;
   const int waves = blockDim.x >> 6;
   const int max_depth = a.max_tree_depth;
   // GLM chains may be shared by the W waves of a block (each evaluates a
