@@ -197,7 +197,7 @@ def _cpu_glm_hmc(x, y, chains, L, eps, transitions, min_ess, budget_s,
 
 
 # ------------------------------------------------ C2 large-batch MFMA HMC
-# HBM bytes per all-chain gradient of glm_grad_mfma<8> at 65536 x 256 x 4096:
+# HBM bytes per all-chain gradient of glm_grad_mfma<4> at 65536 x 256 x 4096:
 # rocprofv3 FETCH_SIZE 265 300 KiB x 2.00 + WRITE_SIZE 32 863 KiB x 1.00 per
 # dispatch, the factors being what the counters read for a 256 MiB device
 # copy (profiles/glm_grad_mfma_logistic_65536x256_counters.md)
@@ -286,7 +286,7 @@ def logistic_65536x256(args, torch, pa):
                    'traffic_what': 'HBM bytes per gradient launch '
                                    '(FETCH_SIZE + WRITE_SIZE, '
                                    'copy-calibrated); X and X^T are 64 MiB',
-                   'kernel': 'glm_grad_mfma<8> + mfma_chain_step (sampling '
+                   'kernel': 'glm_grad_mfma<4> + mfma_chain_step (sampling '
                              'launch, all 1000 transitions)',
                    'algorithmic_flop_per_gradient': flop_grad,
                    'executed_mfma_flop_per_gradient': 2 * flop_grad,
