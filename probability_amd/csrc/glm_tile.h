@@ -192,43 +192,37 @@ __device__ __attribute__((always_inline)) inline void glm_tile_rows(
 #pragma unroll
     for (int s = 0; s < S; ++s)
       *(lptr<Q>)(rows + m * P + 16 * s + 4 * g) = xv[s];
-    // Float32 logits are summed in eight parts (two sets of slabs, each step t
-    // apart): one chain of additions over all columns doubles their rounding
-    // error, and a linear model's residual is a small difference of them.
-    // Relative error of its gradient against float64 at 8192 x 128: one chain
-    // 2.8e-6, four parts 1.5e-6, eight 1.2e-6 (the per-chain pass 1.2e-6);
-    // sixteen parts spill (8192 x 128, 2048 chains 95 -> 126 us).
+    // Logits are summed in four parts (each step t apart), or eight (two sets
+    // of slabs as well): one chain of additions over all columns doubles their
+    // rounding error, and a linear model's residual is a small difference of
+    // them.  Relative error of its gradient, float32 at 8192 x 128 against
+    // float64: one chain 2.8e-6, four parts 1.5e-6, eight 1.2e-6 (the per-chain
+    // pass 1.2e-6); sixteen parts spill (8192 x 128, 2048 chains 95 -> 126 us).
+    // Float64 at 1024 to 1300 rows near the mode, one chain / four / eight
+    // parts, rms error against extended precision over the per-chain pass's:
+    // 127 columns 1.98 / 1.07 / 0.87, 96 columns 1.50 / 0.89 / 0.75, 64 columns
+    // 1.55 / 0.92 / 0.78; so eight from 97 columns on.  (8000 x 127, 1000
+    // chains 130 / 131 / 141 us, where eight spill; 4000 x 64, 1000 chains 50 /
+    // 49 / 65.)
+    constexpr int kSets = S < (sizeof(T) == 4 ? 2 : 7) ? 1 : 2;
     Q lg[NG];
-    if constexpr (sizeof(T) == 4) {
-      constexpr int kSets = S < 2 ? 1 : 2;
 #pragma unroll
-      for (int h = 0; h < kSets; ++h) {
-        Q part[4][NG];
+    for (int h = 0; h < kSets; ++h) {
+      Q part[4][NG];
 #pragma unroll
-        for (int s = h; s < S; s += kSets)
-#pragma unroll
-          for (int t = 0; t < 4; ++t)
-#pragma unroll
-            for (int j = 0; j < NG; ++j)
-              part[t][j] = mfma16x4(
-                  xv[s][t], beta[j][s][t],
-                  s == h ? Q{T(0), T(0), T(0), T(0)} : part[t][j]);
-#pragma unroll
-        for (int j = 0; j < NG; ++j) {
-          const Q sum = (part[0][j] + part[1][j]) + (part[2][j] + part[3][j]);
-          lg[j] = h == 0 ? sum : lg[j] + sum;
-        }
-      }
-    } else {
-#pragma unroll
-      for (int j = 0; j < NG; ++j) lg[j] = Q{T(0), T(0), T(0), T(0)};
-#pragma unroll
-      for (int s = 0; s < S; ++s)
+      for (int s = h; s < S; s += kSets)
 #pragma unroll
         for (int t = 0; t < 4; ++t)
 #pragma unroll
           for (int j = 0; j < NG; ++j)
-            lg[j] = mfma16x4(xv[s][t], beta[j][s][t], lg[j]);
+            part[t][j] = mfma16x4(
+                xv[s][t], beta[j][s][t],
+                s == h ? Q{T(0), T(0), T(0), T(0)} : part[t][j]);
+#pragma unroll
+      for (int j = 0; j < NG; ++j) {
+        const Q sum = (part[0][j] + part[1][j]) + (part[2][j] + part[3][j]);
+        lg[j] = h == 0 ? sum : lg[j] + sum;
+      }
     }
     T yc[4];
 #pragma unroll
