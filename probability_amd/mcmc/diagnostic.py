@@ -11,6 +11,7 @@ everything else with torch.
 
 import math
 
+import numpy as np
 import torch
 
 from probability_amd import _lib
@@ -117,7 +118,12 @@ def _flatten_chain_dims(states, cross_chain_dims):
 
 
 def _ess_one(states, cross_chain_dims, filter_threshold):
-  if cross_chain_dims is not None and _on_device(states) and states.dim() > 1:
+  # the kernel takes one threshold for all dimensions; a tensor that
+  # broadcasts over them (or lies on the GPU) goes to the torch form
+  number = filter_threshold is None or isinstance(
+      filter_threshold, (int, float, np.integer, np.floating))
+  if (cross_chain_dims is not None and number and _on_device(states) and
+      states.dim() > 1):
     x = _flatten_chain_dims(states, cross_chain_dims)
     if 1 <= x.shape[0] <= _MAX_DRAWS and x.shape[1] >= 2 and x.numel() > 0:
       return _ess_device(x, filter_threshold)
