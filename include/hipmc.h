@@ -612,7 +612,7 @@ int hipmc_effective_sample_size(int32_t dtype, int64_t n, int64_t chains,
  * halves of n / 2 draws as chains (an odd last draw is left out).  At least
  * two draws per half.  out: float64 [dims]; ws_sums: float64
  * [chunks, split ? 2 : 1, 2, chains * dims], `chunks` the time chunks whose
- * partial sums are added in order.  Replaces potential_scale_reduction
+ * means and variances are merged in order.  Replaces potential_scale_reduction
  * (mcmc/diagnostic.py:476-568).
  */
 int hipmc_potential_scale_reduction(int32_t dtype, int64_t n, int64_t chains,

@@ -77,10 +77,13 @@ def _rhat_device(state, independent_chain_ndims, split_chains):
   x = _series(state, independent_chain_ndims)
   n, c, d = x.shape
   halves = 2 if split_chains else 1
-  # time chunks so that about 2048 blocks of 64 series run, each with at
-  # least 32 draws
-  blocks = halves * (-(-(c * d) // 64))
-  chunks = max(1, min(2048 // blocks, (n // halves) // 32))
+  # a block takes up to 64 adjacent series, its other threads 16 draws at a
+  # time; time chunks so that about 2048 blocks run, none with less than one
+  # such step
+  width = min(64, 1 << (c * d - 1).bit_length())
+  blocks = halves * -(-(c * d) // width)
+  step = 16 * (256 // width)
+  chunks = max(1, min(2048 // blocks, 512, -(-(n // halves) // step)))
   sums = torch.empty((chunks, halves, 2, c * d), dtype=torch.float64,
                      device=x.device)
   out = torch.empty(d, dtype=torch.float64, device=x.device)
