@@ -504,54 +504,138 @@ __global__ void __launch_bounds__(256)
   }
 }
 
-// One block per dimension: with the mean and unbiased variance of each of the
-// m = halves * chains series of h draws, w the mean of the variances and b
-// the unbiased variance of the means,
+// How rhat_finish shares a dimension's m series out.
+struct RhatShare {
+  int threads;    // of a block
+  int share_log;  // log2 of a block's threads on one dimension
+  int splits;     // blocks on one dimension
+};
+
+__device__ inline double rhat_of(const Moments& means, double var, int m,
+                                 double h) {
+  const double w = var / (double)m;
+  const double s2 = (h - 1.0) / h * w + means.m2 / ((double)m - 1.0);
+  return ((double)m + 1.0) / (double)m * s2 / w - (h - 1.0) / ((double)m * h);
+}
+
+// With the mean and unbiased variance of each of a dimension's m = halves *
+// chains series of h draws, w the mean of the variances and b the unbiased
+// variance of the means,
 //   s2 = (h - 1) / h w + b,  R-hat = (m + 1) / m s2 / w - (h - 1) / (m h).
-__global__ void __launch_bounds__(256)
-    rhat_finish(const double* __restrict__ sums, int h, int halves, int chains,
-                int dims, int chunk, int chunks, double* __restrict__ out) {
-  __shared__ double red[3][256];
-  const int d = blockIdx.x;
-  const int tid = threadIdx.x;
+// Block (adjacent dimensions, range of series).  With several ranges a block
+// leaves its sums in place of its range's first two series (no other block
+// reads them) for rhat_combine.
+__global__ void __launch_bounds__(1024)
+    rhat_finish(double* sums, int h, int halves, int chains, int dims,
+                int chunk, int chunks, RhatShare share,
+                double* __restrict__ out) {
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  double* red = (double*)smem_raw;  // 4 x threads
+  const int tid = threadIdx.x, nt = blockDim.x;
+  const int width = nt >> share.share_log;
+  const int part = tid / width, parts = 1 << share.share_log;
+  const int64_t d = (int64_t)blockIdx.x * width + (tid - part * width);
   const int64_t series = (int64_t)chains * dims;
   const int m = halves * chains;
+  const int per = (m + share.splits - 1) / share.splits;
+  const int i0 = blockIdx.y * per, i1 = min(m, i0 + per);
   const double hn = (double)h;
-  Moments means{0.0, 0.0, 0.0};
-  double var = 0.0, none = 0.0;
-  for (int i = tid; i < m; i += 256) {
+  auto row = [&](int i) {  // of chunk 0
     const int half = i / chains, c = i - half * chains;
-    const double* p =
-        sums + (size_t)half * 2 * series + (int64_t)c * dims + d;
-    Moments a{0.0, 0.0, 0.0};
+    return sums + (size_t)half * 2 * series + (int64_t)c * dims + d;
+  };
+  Moments means{0.0, 0.0, 0.0};
+  double var = 0.0;
+  if (d < dims) {
+    if (chunks == 1) {
 #pragma unroll 8
-    for (int z = 0; z < chunks; ++z, p += (size_t)halves * 2 * series) {
-      const int n = min(chunk, h - z * chunk);
-      a = merge(a, Moments{(double)(n > 0 ? n : 0), p[0], p[series]});
+      for (int i = i0 + part; i < i1; i += parts) {
+        const double* p = row(i);
+        var += p[series] / (hn - 1.0);
+        means = merge(means, Moments{1.0, p[0], 0.0});
+      }
+    } else {
+      for (int i = i0 + part; i < i1; i += parts) {
+        const double* p = row(i);
+        Moments a{0.0, 0.0, 0.0};
+#pragma unroll 8
+        for (int z = 0; z < chunks; ++z, p += (size_t)halves * 2 * series) {
+          const int n = min(chunk, h - z * chunk);
+          a = merge(a, Moments{(double)(n > 0 ? n : 0), p[0], p[series]});
+        }
+        var += a.m2 / (hn - 1.0);
+        means = merge(means, Moments{1.0, a.mean, 0.0});
+      }
     }
-    var += a.m2 / (hn - 1.0);
-    means = merge(means, Moments{1.0, a.mean, 0.0});
   }
-  block_sum2(var, none, &red[0][0]);
-  red[0][tid] = means.n;
-  red[1][tid] = means.mean;
-  red[2][tid] = means.m2;
-  for (int k = 128; k >= 1; k >>= 1) {
+  for (int k = nt >> 1; k >= width; k >>= 1) {
+    red[tid] = means.n;
+    red[nt + tid] = means.mean;
+    red[2 * nt + tid] = means.m2;
+    red[3 * nt + tid] = var;
     __syncthreads();
     if (tid < k) {
-      means = merge(means, Moments{red[0][tid + k], red[1][tid + k],
-                                   red[2][tid + k]});
-      red[0][tid] = means.n;
-      red[1][tid] = means.mean;
-      red[2][tid] = means.m2;
+      const int o = tid + k;
+      means = merge(means, Moments{red[o], red[nt + o], red[2 * nt + o]});
+      var += red[3 * nt + o];
     }
+    __syncthreads();
   }
-  if (tid == 0) {
-    const double w = var / (double)m;
-    const double s2 = (hn - 1.0) / hn * w + means.m2 / ((double)m - 1.0);
-    out[d] = ((double)m + 1.0) / (double)m * s2 / w -
-             (hn - 1.0) / ((double)m * hn);
+  if (part != 0 || d >= dims) return;
+  if (share.splits == 1) {
+    out[d] = rhat_of(means, var, m, hn);
+  } else {
+    double* p = row(i0);
+    p[0] = means.mean;
+    p[series] = means.m2;
+    row(i0 + 1)[0] = var;
   }
+}
+
+// One thread per dimension: the ranges of rhat_finish in order.
+__global__ void __launch_bounds__(256)
+    rhat_combine(const double* __restrict__ sums, int h, int halves, int chains,
+                 int dims, int splits, double* __restrict__ out) {
+  const int64_t d = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (d >= dims) return;
+  const int64_t series = (int64_t)chains * dims;
+  const int m = halves * chains;
+  const int per = (m + splits - 1) / splits;
+  auto row = [&](int i) {
+    const int half = i / chains, c = i - half * chains;
+    return sums + (size_t)half * 2 * series + (int64_t)c * dims + d;
+  };
+  Moments means{0.0, 0.0, 0.0};
+  double var = 0.0;
+#pragma unroll 8
+  for (int y = 0; y < splits; ++y) {
+    const int i0 = y * per;
+    const double* p = row(i0);
+    means = merge(means,
+                  Moments{(double)(min(m, i0 + per) - i0), p[0], p[series]});
+    var += row(i0 + 1)[0];
+  }
+  out[d] = rhat_of(means, var, m, (double)h);
+}
+
+// One thread per series, up to a block of adjacent dimensions, but fewer (down
+// to one per eight series) where the dimensions alone fill the GPU; several
+// blocks where a dimension has thousands of series.  Each range has at least
+// two series.  Split R-hat, us, torch form / one block of 256 threads per
+// dimension, whatever its series / now: 65 draws, 2 chains, 1e6 dimensions 881 /
+// 1642 / 230; 65 draws, 250000 chains, 1 dimension 128 / 354 / 62; 1000 draws,
+// 100000 chains, 1 dimension 684 / 762 / 111.
+RhatShare rhat_share(int m, int dims) {
+  int log = 0;
+  while (log < 10 && (1 << log) < m) ++log;
+  while (log > 0 && ((int64_t)dims << log) > (1 << 17) && m < (8 << log)) --log;
+  if (log <= 8) return RhatShare{256, log, 1};
+  for (int w = 1; w < 8 && w < dims; w <<= 1) --log;
+  int splits = 1;
+  while (splits < 32 && m >= (2 << log) * 2 * splits &&
+         ((int64_t)dims << log) * splits < (1 << 17))
+    splits <<= 1;
+  return RhatShare{1024, log, splits};
 }
 
 template <typename F>
@@ -617,8 +701,16 @@ int rhat_run(int h, int halves, int chains, int dims, int64_t sn, int64_t sc,
                           chunks),
                      dim3(256), 0, s, x, h, chains, dims, sn, sc, sd, chunk, w,
                      sums);
-  hipLaunchKernelGGL(rhat_finish, dim3(dims), dim3(256), 0, s, sums, h, halves,
-                     chains, dims, chunk, chunks, out);
+  const RhatShare share = rhat_share(halves * chains, dims);
+  const int width = share.threads >> share.share_log;
+  hipLaunchKernelGGL(rhat_finish,
+                     dim3((dims + width - 1) / width, share.splits),
+                     dim3(share.threads), 4 * share.threads * sizeof(double),
+                     s, sums, h, halves, chains, dims, chunk, chunks, share,
+                     out);
+  if (share.splits > 1)
+    hipLaunchKernelGGL(rhat_combine, dim3((dims + 255) / 256), dim3(256), 0, s,
+                       sums, h, halves, chains, dims, share.splits, out);
   return hip_check(hipGetLastError(), "rhat launch");
 }
 
@@ -683,6 +775,9 @@ int hipmc_potential_scale_reduction(int32_t dtype, int64_t n, int64_t chains,
     return fail(HIPMC_E_UNSUPPORTED, "rhat: too many chains");
   if (chunks < 1 || chunks > 65535)
     return fail(HIPMC_E_INVALID, "rhat: chunks must be in [1, 65535]");
+  // a grid holds fewer than 2^32 threads: 256 per 64 series
+  if (chains * dims >= 1 << 30)
+    return fail(HIPMC_E_UNSUPPORTED, "rhat: too many series");
   const int h = (int)(n / halves);
   hipStream_t s = as_stream(stream);
   if (dtype == HIPMC_F32)

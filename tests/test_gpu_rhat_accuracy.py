@@ -55,3 +55,46 @@ def test_chains_that_never_move_have_no_variance(dtype, n, c, d, value):
   x[:, 0] *= 2  # variance between the chains only
   assert bool(torch.isinf(pdiag.potential_scale_reduction(
       x, split_chains=True)).all())
+
+
+@pytest.mark.parametrize('split', [True, False])
+@pytest.mark.parametrize('n,c,d', [
+    (50, 1, 300), (50, 2, 1), (50, 3, 5), (41, 700, 1), (50, 6000, 1),
+    (41, 6001, 9), (45, 20000, 12), (41, 130001, 1), (50, 3, 20001),
+    (41, 2, 300001), (3000, 5, 1), (3000, 2100, 1), (400, 300, 17)])
+def test_every_division_of_the_series_matches(n, c, d, split):
+  """One thread to several blocks on a dimension, one to many time chunks."""
+  r = np.random.default_rng(n + c + d)
+  x = (r.normal(size=(n, c, d)) + r.normal(size=(c, 1)) + 5).astype(np.float32)
+  if not split and c == 1:
+    return  # no variance between chains
+  got = pdiag.potential_scale_reduction(torch.as_tensor(x, device='cuda'),
+                                        split_chains=split).cpu().numpy()
+  want = _rhat(x, split)
+  assert got.shape == want.shape
+  # as above; up to 260002 series are merged, in at most 300 steps in a row
+  assert np.abs((got - want) / want).max() <= 1e-13
+
+
+def test_more_dimensions_than_a_grid_of_blocks():
+  """2^24 + 3 dimensions: a block of 256 threads for each would be a grid of
+  2^32 threads, one more than is taken."""
+  n, c, d = 41, 2, (1 << 24) + 3
+  g = torch.Generator(device='cuda')
+  g.manual_seed(0)
+  x = torch.randn((n, c, d), generator=g, device='cuda')
+  got = pdiag.potential_scale_reduction(x)
+  at = torch.tensor([0, 1, 1 << 23, (1 << 24) - 1, 1 << 24, d - 1],
+                    device='cuda')
+  want = _rhat(x[:, :, at].cpu().numpy(), False)
+  assert got.shape == (d,)
+  assert np.abs((got[at].cpu().numpy() - want) / want).max() <= 1e-13
+
+
+def test_the_kernels_limits_are_those_of_their_grids():
+  x = torch.empty(1)
+  takes = lambda *shape: pdiag._rhat_takes(x.expand(shape), 1)
+  assert takes(4, 2, 1) and takes(41, 2, 1 << 28) and not takes(41, 2, 1 << 29)
+  assert not takes(41, (1 << 29) + 1, 1) and not takes((1 << 30) + 1, 1, 1)
+  assert takes(40, 2, 1000) and not takes(40, 2, 250000) and takes(41, 2, 250000)
+  assert not pdiag._rhat_takes(x.expand(50, 2), 2)
