@@ -40,6 +40,21 @@ def _on_device(x):
           not torch.compiler.is_compiling())
 
 
+def _ess_takes(n, c, d):
+  """Whether the ESS of n draws of c chains of d dimensions is the kernels':
+  within their limits (a grid holds fewer than 2^32 threads), and not where the
+  torch form is faster: few draws, since a block's fixed work per pair of chains
+  is that of 64 threads, and short series of very many chains, which few blocks
+  share.  us, torch form / kernels: 4 draws, 25000 x 3 series 241 / 252, 2 x
+  1000000 1012 / 1665; 8 draws, 2000 x 500 1113 / 1131, 100000 x 1 275 / 690; 17
+  draws, 20000 x 50 4248 / 1344, 250000 x 1 1383 / 1684; 65 draws, 250000 x 1
+  7130 / 1812."""
+  if not (n <= _MAX_DRAWS and 2 <= c <= 1 << 30 and c * d < 1 << 30 and
+          d * max(64, n // 4) < 1 << 32):
+    return False
+  return n > 64 or c * d <= 50000 or (n > 8 and c <= 65536)
+
+
 def _rhat_takes(x, chain_axes):
   """Whether R-hat of draws x [n, chain axes..., ...] is the kernels': within
   their limits, and not for few draws of very many series, where a pass over
@@ -144,7 +159,7 @@ def _ess_one(states, cross_chain_dims, filter_threshold):
   if (cross_chain_dims is not None and number and _on_device(states) and
       states.dim() > 1):
     x = _flatten_chain_dims(states, cross_chain_dims)
-    if 1 <= x.shape[0] <= _MAX_DRAWS and x.shape[1] >= 2 and x.numel() > 0:
+    if x.numel() > 0 and _ess_takes(*_series(x, 1).shape):
       return _ess_device(x, filter_threshold)
   states = _as64(states)
   if cross_chain_dims is not None:

@@ -36,3 +36,25 @@ def test_threshold_tensors_broadcast_over_the_dimensions(where):
       for i, t in enumerate(th)])
   # the forms' transforms differ by rounding (see the size tests' bound)
   torch.testing.assert_close(got, want, rtol=1e-9, atol=0)
+
+
+def test_ess_rule_and_limits():
+  takes = pdiag._ess_takes
+  assert takes(1, 2, 1) and takes(4096, 2, 1) and not takes(4097, 2, 1)
+  assert not takes(100, 1, 5) and not takes(100, 1 << 29, 2)
+  assert takes(8, 2, 25000) and not takes(8, 2, 25001) and takes(9, 2, 25001)
+  assert takes(64, 65536, 1) and not takes(64, 65537, 1) and takes(65, 65537, 1)
+  assert takes(4096, 2, (1 << 22) - 1) and not takes(4096, 2, 1 << 22)
+
+
+@pytest.mark.parametrize('n,c,d', [(4, 2, 25001), (8, 7000, 9), (8, 2, 25000),
+                                   (9, 2, 30000), (64, 70000, 1), (70, 70000, 1)])
+def test_ess_on_both_sides_of_the_rule(n, c, d):
+  """Against the same draws in float64 on the CPU, which the kernels never
+  take (tolerance as above)."""
+  x = _draws(n, c, d, n)
+  want = pdiag.effective_sample_size(x.double().cpu(), cross_chain_dims=1,
+                                     filter_threshold=None)
+  got = pdiag.effective_sample_size(x, cross_chain_dims=1,
+                                    filter_threshold=None)
+  torch.testing.assert_close(1 / got.cpu(), 1 / want, rtol=1e-9, atol=1e-12)
