@@ -112,13 +112,24 @@ def flat_inputs(spec, parts, tlp, grads):
   return state, t.reshape(-1), grad
 
 
+def choose_lists(accepted, pairs):
+  """choose_rows of several (proposed, current) pairs of lists, together where
+  each pair's lists are as long as each other."""
+  if any(len(p) != len(c) for p, c in pairs):
+    return [mcmc_util.choose(accepted, list(p), list(c)) for p, c in pairs]
+  rows = iter(choose_rows(accepted, [v for p, _ in pairs for v in p],
+                          [v for _, c in pairs for v in c]))
+  return [[next(rows) for _ in p] for p, _ in pairs]
+
+
 def choose_rows(accepted, proposed, current):
-  """[torch.where(accepted, p, c)] of lists of per-chain tensors, in one
-  launch where they are plain tensors of one type and shape on the current
-  GPU."""
+  """[torch.where(accepted, p, c)] of lists of per-chain tensors (as long as
+  the shorter one), in one launch where they are equally many plain tensors of
+  one type and shape on the current GPU."""
   n = accepted.numel()
   first = proposed[0]
-  if (n == 0 or len(proposed) > _lib.MAX_COPY_BLOCKS or not first.is_cuda or
+  if (n == 0 or len(proposed) != len(current) or
+      len(proposed) > _lib.MAX_COPY_BLOCKS or not first.is_cuda or
       first.device.index != torch.cuda.current_device() or
       first.element_size() not in (4, 8) or
       any(not isinstance(c, torch.Tensor) or c.requires_grad or

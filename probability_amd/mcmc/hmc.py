@@ -219,18 +219,16 @@ class HamiltonianMonteCarlo(kernel_base.TransitionKernel):
         initial_momentum=spec.unpack_state(p0, cs),
         final_momentum=spec.unpack_state(p1, cs),
         seed=samplers.first_child(seed))
-    k = len(proposed_results.initial_momentum)
-    chosen = _runner.choose_rows(
-        accepted, [proposed_results.log_acceptance_correction,
-                   *proposed_results.initial_momentum,
-                   *proposed_results.final_momentum],
-        [acc.log_acceptance_correction, *_as_parts(acc.initial_momentum),
-         *_as_parts(acc.final_momentum)])
+    (correction,), p_initial, p_final = _runner.choose_lists(accepted, [
+        ([proposed_results.log_acceptance_correction],
+         [acc.log_acceptance_correction]),
+        (proposed_results.initial_momentum, _as_parts(acc.initial_momentum)),
+        (proposed_results.final_momentum, _as_parts(acc.final_momentum))])
     new_acc = acc._replace(
-        log_acceptance_correction=chosen[0],
+        log_acceptance_correction=correction,
         target_log_prob=tlp.reshape(cs),
         grads_target_log_prob=spec.unpack_state(grad, cs),
-        initial_momentum=chosen[1:1 + k], final_momentum=chosen[1 + k:],
+        initial_momentum=p_initial, final_momentum=p_final,
         seed=[])
     results = mh.MetropolisHastingsKernelResults(
         accepted_results=new_acc, is_accepted=accepted,
