@@ -117,7 +117,7 @@ class PosteriorBatch:
     if fams == {1}:
       cols = max(d - (s.kind == _lib.TARGET_LINEAR)
                  for s, d in zip(self.specs, self.dims))
-      self._tiles = glm_tile.BatchTiles([s.base.n_obs for s in self.specs],
+      self._tiles = glm_tile.BatchTiles([_rows(s) for s in self.specs],
                                         cols, self.num_chains, offs,
                                         self.dtype, self.device)
     g = int(chains_per_block or 1)
@@ -197,6 +197,13 @@ class PosteriorBatch:
             for i in range(self.n_problems)]
 
 
+def _rows(spec):
+  """Observations of a regression spec, or of the one it transforms."""
+  while spec.base is not spec:
+    spec = spec.base
+  return spec.n_obs
+
+
 def _leaf_cost(spec, dtype):
   """Microseconds of one leapfrog of a GLM chain on a CU of its own (eight
   waves): 7 for the trajectory's bookkeeping, and per 1000 rows 0.3 and 2.1
@@ -204,7 +211,7 @@ def _leaf_cost(spec, dtype):
   23.5 at 7038 x 34, 17.9 at 2842 x 118, 27.2 at 4359 x 86 with 64 elements to
   the block)."""
   block = 64 if dtype == torch.float32 else 32
-  return 7.0 + spec.n_obs * (3e-4 + 2.1e-3 * -(-spec.dim // block))
+  return 7.0 + _rows(spec) * (3e-4 + 2.1e-3 * -(-spec.dim // block))
 
 
 def _start_order(cost, num_chains, n_xcd=8):
