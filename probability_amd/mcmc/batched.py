@@ -114,6 +114,7 @@ class PosteriorBatch:
       self.kind = _lib.TARGET_DIAG_NORMAL
     self._tiles = None  # of eval()
     self._order = None  # of start_order()
+    self._streams = set()  # that _keep has seen
     if fams == {1}:
       cols = max(d - (s.kind == _lib.TARGET_LINEAR)
                  for s, d in zip(self.specs, self.dims))
@@ -150,12 +151,29 @@ class PosteriorBatch:
       self._order = (torch.as_tensor(
           _start_order(cost, self.num_chains), device=self.device)
                      if min(cost) < max(cost) else None,)
+      self._streams.clear()
+    self._keep()
     return self._order[0]
+
+  def _keep(self):
+    """Before a launch on the current stream reads the batch's device arrays:
+    should the batch be dropped, their memory is not given out again until that
+    stream's work is done (they were allocated on other streams)."""
+    handle = _lib.stream_handle(self.device)
+    if handle not in self._streams:
+      stream = torch.cuda.current_stream(self.device)
+      for t in (self.table, self.chain_problem, self.chain_local,
+                self.group_start, self._order and self._order[0],
+                self._tiles and self._tiles.table):
+        if t is not None:
+          t.record_stream(stream)
+      self._streams.add(handle)
 
   def eval(self, x):
     """(tlp [C], grad [C, dim_stride]) of every chain at x."""
     if self._tiles is None or self._tiles.table is None:
       return self.eval_chains(x)
+    self._keep()
     tlp = torch.empty(self.n_chains, dtype=self.dtype, device=self.device)
     grad = torch.zeros_like(x)
     self._tiles.evaluate(self, x, tlp, grad)
@@ -164,6 +182,7 @@ class PosteriorBatch:
   def eval_chains(self, x):
     """eval by the samplers' own per-chain pass, whose sums do not depend on
     the batch (a run starts from them, so that its draws do not either)."""
+    self._keep()
     tlp = torch.empty(self.n_chains, dtype=self.dtype, device=self.device)
     grad = torch.zeros_like(x)
     _lib.check(_lib.lib().hipmc_target_eval(
@@ -174,6 +193,7 @@ class PosteriorBatch:
     return tlp, grad
 
   def bijector(self, x, direction, chain_period=0):
+    self._keep()
     out = torch.empty_like(x)
     rows = x.numel() // self.dim_stride
     _lib.check(_lib.lib().hipmc_bijector(
