@@ -21,6 +21,14 @@ def _arrays(batch):
   return out
 
 
+def _use(batch, use, x):
+  if use == 'bijector':
+    return batch.bijector(x, 0)
+  if use == 'order':
+    return batch.start_order().clone()
+  return getattr(batch, use)(x)
+
+
 @pytest.mark.parametrize('use', ['eval', 'eval_chains', 'bijector', 'order'])
 def test_arrays_outlive_another_streams_work(use):
   r = np.random.default_rng(0)
@@ -29,29 +37,25 @@ def test_arrays_outlive_another_streams_work(use):
     x = r.normal(size=(n, d)).astype(np.float32)
     specs.append(ptg.LogisticRegression(
         x, (r.uniform(size=n) < 0.5).astype(np.float32), device='cuda'))
-  batch = batched.PosteriorBatch(specs, num_chains=4, waves_per_chain=4)
+  warm, batch = [batched.PosteriorBatch(specs, num_chains=4, waves_per_chain=4)
+                 for _ in range(2)]
   x = torch.zeros((8, batch.dim_stride), device='cuda')
-  order_on = torch.cuda.Stream()
+  order_on, side = torch.cuda.Stream(), torch.cuda.Stream()
+  with torch.cuda.stream(side):  # whatever the first call of a kind loads
+    torch.cuda._sleep(1000)
+    _use(warm, use, x)
   if use == 'order':  # allocated on a run's stream, read on another run's
     with torch.cuda.stream(order_on):
       assert batch.start_order() is not None
   batch.eval(x)
   torch.cuda.synchronize()
-  side = torch.cuda.Stream()
   with torch.cuda.stream(side):
-    torch.cuda._sleep(200_000_000)  # some 0.1 s
-    if use == 'bijector':
-      got = batch.bijector(x, 0)
-    elif use == 'order':
-      got = batch.start_order().clone()
-    else:
-      got = getattr(batch, use)(x)
+    torch.cuda._sleep(400_000_000)  # some 0.2 s
+    got = _use(batch, use, x)
   sizes = [(t.data_ptr(), t.nbytes) for t in _arrays(batch)]
   del batch
-  streams = [torch.cuda.default_stream(), order_on]
-  taken = set()
-  held = []
-  for s in streams:
+  taken, held = set(), []
+  for s in (torch.cuda.default_stream(), order_on):
     with torch.cuda.stream(s):
       for _, n in sizes:
         for _ in range(8):
