@@ -4,37 +4,47 @@ its workspaces.
 
 The other path is the sampling kernels' own: one chain per wave (up to four
 waves per chain in HMC) passing over X by itself, one launch for a whole
-trajectory.  The tiled one pays two launches per gradient, about 9 to 13 us
-however small the problem.  Where the lines lie, us per evaluation (or per
-leapfrog step) one chain per wave / tiled, logistic regression, MI355X:
+trajectory.  The tiled one pays two launches per gradient, about 9 to 16 us
+however small the problem, and 7 us more of host time per evaluation.  Where
+the lines lie, us per call (evaluations, one after the other) or per leapfrog
+step (four transitions of ten steps in a launch), one chain per wave / tiled,
+MI355X:
 
-  evaluation  float32  256 x 100, 512 chains   11.1 / 13.1
-                       512 x 6,   64 chains    10.7 / 10.1
-                       512 x 30,  512 chains   13.6 / 9.7
-                       8192 x 100, 8 chains     212 / 12
-              float64  256 x 30,  512 chains   10.5 / 12.3
-                       128 x 100, 64 chains    14.8 / 13.0
-  trajectory  float32  2048 x 6,  64 chains     9.9 / 10.6
-                       4096 x 6,  64 chains    17.4 / 11.3
-                       512 x 30,  512 chains   11.3 / 11.4
-                       1024 x 30, 512 chains   20.7 / 11.8
-                       512 x 30,  2048 chains  22.6 / 12.6
-              float64  1024 x 6,  512 chains   12.7 / 13.9
-                       2048 x 6,  64 chains    20.9 / 12.7
-                       1024 x 30, 512 chains   19.3 / 15.0
-                       256 x 100, 64 chains    14.5 / 14.4
-                       256 x 100, 512 chains   29.5 / 15.0
+  evaluation  float32  logistic   512 x 30,  256 chains   12.2 / 17.0
+                                  800 x 30,  1 chain      16.6 / 16.9
+                                  1200 x 8,  1 chain      18.5 / 16.8
+                       linear     512 x 16,  4096 chains  26.4 / 17.1
+                                  800 x 128, 64 chains    20.5 / 18.6
+              float64  logistic   128 x 100, 64 chains    14.5 / 17.2
+                                  512 x 64,  64 chains    24.2 / 18.0
+                       linear     1300 x 30, 1 chain      19.2 / 21.1
+                                  512 x 100, 64 chains    23.7 / 17.1
+  trajectory  float32  logistic   512 x 8,   2000 chains  10.5 / 11.5
+                                  2048 x 8,  256 chains    9.2 / 10.6
+                                  3000 x 30, 256 chains   15.0 / 11.5
+                                  700 x 200, 1000 chains  38.9 / 20.2
+                       linear     1024 x 64, 512 chains   11.1 / 13.9
+                                  2048 x 64, 256 chains    9.1 / 13.6
+                                  3000 x 8,  64 chains    12.5 / 10.1
+              float64  logistic   512 x 64,  256 chains    8.0 / 16.2
+                                  1024 x 64, 256 chains   13.6 / 16.7
+                                  1024 x 30, 512 chains   15.9 / 14.4
+                                  1024 x 100, 64 chains   23.8 / 15.6
+                       linear     2048 x 30, 64 chains     9.5 / 11.6
+                                  3000 x 30, 64 chains    13.0 / 11.9
+  batch       float32  logistic   16 of 128..600 x 30, 16 chains    16.6 / 21.4
+              float64  logistic   256 of 512..2000 x 4, 1 chain     41.0 / 78.7
 
 In float64 a logistic density's exponentials make the per-chain pass up to
-three times as dear as a linear one's (128 x 100, 64 chains, evaluation
-14.8 against 11.6; 1024 x 64, 8 chains, trajectory 24.9 against 9.5), so the
-lines of narrow or short designs hold for logistic ones only.
+three times as dear as a linear one's, so some lines hold for logistic ones
+only.
 """
 
 import numpy as np
 import torch
 
 from probability_amd import _lib
+from probability_amd import tuning
 
 _REGRESSIONS = (_lib.TARGET_LOGISTIC, _lib.TARGET_LINEAR)
 
@@ -53,13 +63,37 @@ def takes_eval(spec, dim, chains):
   n, d = spec.base.n_obs, dim - (kind == _lib.TARGET_LINEAR)
   if d > max_columns(spec.dtype):
     return False
-  return n >= 512 or (spec.dtype == torch.float64 and n * d >= 12000 and
-                      kind == _lib.TARGET_LOGISTIC)
+  if chains >= 4096:
+    return n >= 512
+  if spec.dtype == torch.float32:
+    return n >= (900 if d >= 64 else 1200) or n * d >= 110000
+  if kind == _lib.TARGET_LOGISTIC:
+    return n >= 900 or n * d >= 27000
+  return n >= 1400 or n * d >= 70000
+
+
+# How long the per-chain path's leapfrog is, in passes of a wave over its
+# registers' worth of rows, from where trajectories are tiled: per (float32,
+# logistic) the columns up to which a line holds, the passes, and the same for
+# trajectories of one or two steps, which carry the launch that starts them.
+_PASSES = {
+    (True, True): ((128, 3.0, 4.0), (256, 0.0, 0.0)),
+    (True, False): ((16, 3.0, 3.4), (32, 2.2, 0.0), (64, 3.4, 3.4),
+                    (128, 2.2, 0.0), (256, 0.0, 0.0)),
+    (False, True): ((16, 3.2, 0.0), (32, 0.0, 0.0), (64, 2.5, 2.5),
+                    (128, 1.2, 0.0)),
+    (False, False): ((16, 2.5, 0.0), (32, 3.2, 0.0), (64, 4.5, 0.0),
+                     (128, 0.0, 0.0)),
+}
 
 
 def takes_trajectory(spec, dim, chains, leapfrogs):
-  """Whether HMC trajectories of `chains` chains are tiled.  Trajectories of
-  one or two steps carry the launch that starts them as well."""
+  """Whether HMC trajectories of `chains` chains are tiled: from the rows and
+  chains on that are worth the launches of trajectories, and where the
+  per-chain path takes more than a few passes.  Its waves share a chain's
+  rows (256 a pass, 128 of float64 rows of more than 32 columns); more waves
+  than the 1024 that run at once take proportionally longer in float64, which
+  is bound by arithmetic, and less in float32."""
   kind = spec.kind
   if kind not in _REGRESSIONS or chains < 1 or leapfrogs < 1:
     return False
@@ -67,13 +101,22 @@ def takes_trajectory(spec, dim, chains, leapfrogs):
   if d > max_columns(spec.dtype):
     return False
   f = 1 if leapfrogs > 2 else 2
-  if spec.dtype == torch.float32:
-    return n >= 3000 * f or (n >= 512 and n * chains >= 500000 * f)
-  if n >= 2048 * f:
-    return True
-  if d >= 64 and kind == _lib.TARGET_LOGISTIC:
-    return n >= 1024 * f or n * chains >= 131072 * f
-  return n >= 512 and n * chains >= (500000 if d > 16 else 1000000) * f
+  f32, logistic = spec.dtype == torch.float32, kind == _lib.TARGET_LOGISTIC
+  if f32:
+    long = n >= 3000 * f or (
+        n >= 512 and n * chains >= (500000 if n >= 700 else 700000) * f)
+  elif d >= 64 and logistic:
+    long = n >= 1024 * f or n * chains >= 131072 * f
+  else:
+    long = n >= 2048 * f or (
+        n >= 512 and n * chains >= (500000 if d > 16 else 1000000) * f)
+  if not long:
+    return False
+  waves = min(4, tuning.glm_waves(kind, n, dim, chains, 'hmc', spec.dtype))
+  passes = -(-n // ((256 if f32 or d <= 32 else 128) * waves))
+  passes *= max(1.0, chains * waves / 1024) ** (0.6 if f32 else 1.0)
+  least = next(v for v in _PASSES[f32, logistic] if d <= v[0])
+  return passes >= least[f]
 
 
 def dim_x(spec):
@@ -123,13 +166,25 @@ class BatchTiles:
     chains[i] chains from row offsets[i]."""
     self.table = None
     rows, chains = np.asarray(rows), np.asarray(chains)
-    if (cols > max_columns(dtype) or rows.max() < 512 or chains.min() < 1):
+    n, c = int(rows.max()), int(chains.sum())
+    if cols > max_columns(dtype) or n < 512 or chains.min() < 1:
+      return
+    # the per-chain pass takes as long as the longest problem's rows, until
+    # the chains fill the GPU
+    if c < 4096 and n < 1300 and n * cols < (
+        110000 if dtype == torch.float32 else 70000):
       return
     slabs = -(-cols // 16)
     wide = slabs <= (8 if dtype == torch.float32 else 4)
     ct = 32 if wide and chains.max() > 16 else 16
     tiles = -(-chains // ct)
     n_tiles = int(tiles.sum())
+    # many tiles of a few chains each are mostly empty (a narrow float64
+    # design's per-chain pass is the cheaper: 512 of 128..4000 x 4, 8 chains 183
+    # us, tiled 214)
+    fill = 0.75 * ct if dtype == torch.float64 and cols <= 16 else 8
+    if n_tiles > 128 and c < fill * n_tiles:
+      return
     # rows per range, a multiple of 64: sum of tiles * ceil(rows / per) is at
     # most the sum of tiles * rows over per, plus the tiles
     per = -(-int((tiles * rows).sum()) // (64 * max(768 - n_tiles, 1))) * 64
