@@ -936,7 +936,8 @@ __global__ void __launch_bounds__(256)
                 int n_chains, int dim_stride, const T* x, T* out_tlp,
                 T* out_grad) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  // (not made a scalar: 500 x 100, 4000 chains 43.5 us, as a scalar 47.5)
+  const int wave = threadIdx.x >> 6;
   const int waves = blockDim.x >> 6;
   const int c = blockIdx.x * waves + wave;
   if (c >= n_chains) return;
