@@ -680,6 +680,17 @@ struct ChainQueue {
   }
 };
 
+// Whether the queue has a kernel of its own beside the one of other launches.
+// Float64 regressions of up to 320 elements spill less without its loop (4
+// slots 822 registers, with it 1144): 100 x 200, 4000 chains, one transition
+// 14.3 ms, with it 16.4; 20 x 130 1.24 and 1.69.  Eight slots spill less with
+// it (200 x 400, 1024 chains 21.8 ms, without 23.9), float32 ones hardly
+// differ.
+template <typename T, int K, int FAM>
+constexpr bool nuts_queue_apart() {
+  return FAM == kFamilyGlm && sizeof(T) == 8 && K < 8;
+}
+
 // Between its gradients a leaf is bound by the instructions its wave issues,
 // four cycles each and one after the other (in every wave of a shared chain).
 // The leaf's sums are reduced in pairs and fours that share their last stages,
@@ -692,7 +703,9 @@ struct ChainQueue {
 // waves per SIMD (the register budget that allows) and blocks of up to
 // eight waves (one chain shared by a whole CU); the other families keep one
 // wave per SIMD and every register for the leaf's latency.
-template <typename T, int K, int FAM>
+// QUEUE = false: without the queue's loop around the chain, which costs the
+// float64 kernels registers (nuts_queue_apart).
+template <typename T, int K, int FAM, bool QUEUE>
 __global__ void __launch_bounds__(FAM == kFamilyGlm ? 512 : 256)
     __attribute__((amdgpu_waves_per_eu(FAM == kFamilyGlm ? 2 : 1)))
     nuts_kernel(hipmc_run_args a, int32_t* queue, const int32_t* order) {
@@ -711,7 +724,7 @@ __global__ void __launch_bounds__(FAM == kFamilyGlm ? 512 : 256)
   // share of the rows, the partial sums meet in LDS, every wave runs the
   // same control flow on the same values); otherwise a wave per chain.
   const int W = waves_per_chain<FAM>(a);
-  const bool queued = FAM == kFamilyGlm && W > 1 && queue != nullptr;
+  const bool queued = QUEUE && W > 1 && queue != nullptr;
   ChainQueue cq;
   int c = xcd_block(blockIdx.x, gridDim.x);
   if (W == 1) c = c * waves + wave;

@@ -96,17 +96,20 @@ int launch_nuts(const hipmc_run_args& a0, int32_t* queue,
   int W = waves_per_chain<FAM>(a);
   while (W > 1 && shared_bytes(W) > (size_t)kMaxLdsSharedChain) --W;
   a.waves_per_chain = W;
+  auto* const from_queue = &nuts_kernel<T, K, FAM, FAM == kFamilyGlm>;
+  auto* const plain = &nuts_kernel<
+      T, K, FAM, FAM == kFamilyGlm && !nuts_queue_apart<T, K, FAM>()>;
   if (W > 1) {
     const size_t bytes = shared_bytes(W);
-    const int rc = allow_lds(&nuts_kernel<T, K, FAM>, bytes);
-    if (rc != HIPMC_OK) return rc;
     // blocks of 8 waves share a chain at two waves per SIMD, so 8 / W blocks
     // fit a CU; more chains than that are handed out as blocks get ready
     const int resident = device_cus() * (8 / W);
     if (a.n_chains <= resident) queue = nullptr;
-    hipLaunchKernelGGL((nuts_kernel<T, K, FAM>),
-                       dim3(queue ? resident : a.n_chains), dim3(64 * W),
-                       bytes, s, a, queue, order);
+    auto* const kernel = queue ? from_queue : plain;
+    const int rc = allow_lds(kernel, bytes);
+    if (rc != HIPMC_OK) return rc;
+    hipLaunchKernelGGL(kernel, dim3(queue ? resident : a.n_chains),
+                       dim3(64 * W), bytes, s, a, queue, order);
     return hip_check(hipGetLastError(), "nuts_kernel launch");
   }
   const size_t per_wave = (cl + wl) * sizeof(T);
@@ -117,16 +120,16 @@ int launch_nuts(const hipmc_run_args& a0, int32_t* queue,
       return fail(HIPMC_E_UNSUPPORTED,
                   "U-turn memory does not fit in LDS (lower max_tree_depth "
                   "or use float32)");
-    const int rc = allow_lds(&nuts_kernel<T, K, FAM>, per_wave);
+    const int rc = allow_lds(plain, per_wave);
     if (rc != HIPMC_OK) return rc;
-    hipLaunchKernelGGL((nuts_kernel<T, K, FAM>), dim3(a.n_chains), dim3(64),
-                       per_wave, s, a, (int32_t*)nullptr, (const int32_t*)nullptr);
+    hipLaunchKernelGGL(plain, dim3(a.n_chains), dim3(64), per_wave, s, a,
+                       (int32_t*)nullptr, (const int32_t*)nullptr);
     return hip_check(hipGetLastError(), "nuts_kernel launch");
   }
   const int w = waves_for_lds(per_wave);
   const int blocks = (a.n_chains + w - 1) / w;
-  hipLaunchKernelGGL((nuts_kernel<T, K, FAM>), dim3(blocks), dim3(64 * w),
-                     per_wave * w, s, a, (int32_t*)nullptr, (const int32_t*)nullptr);
+  hipLaunchKernelGGL(plain, dim3(blocks), dim3(64 * w), per_wave * w, s, a,
+                     (int32_t*)nullptr, (const int32_t*)nullptr);
   return hip_check(hipGetLastError(), "nuts_kernel launch");
 }
 
