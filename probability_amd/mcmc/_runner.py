@@ -115,11 +115,18 @@ def flat_inputs(spec, parts, tlp, grads):
 def choose_lists(accepted, pairs):
   """choose_rows of several (proposed, current) pairs of lists, together where
   each pair's lists are as long as each other."""
-  if any(len(p) != len(c) for p, c in pairs):
-    return [mcmc_util.choose(accepted, list(p), list(c)) for p, c in pairs]
-  rows = iter(choose_rows(accepted, [v for p, _ in pairs for v in p],
-                          [v for _, c in pairs for v in c]))
-  return [[next(rows) for _ in p] for p, _ in pairs]
+  proposed, current = [], []
+  for p, c in pairs:
+    if len(p) != len(c):
+      return [mcmc_util.choose(accepted, list(p), list(c)) for p, c in pairs]
+    proposed += p
+    current += c
+  rows = choose_rows(accepted, proposed, current)
+  out, at = [], 0
+  for p, _ in pairs:
+    out.append(rows[at:at + len(p)])
+    at += len(p)
+  return out
 
 
 def choose_rows(accepted, proposed, current):
