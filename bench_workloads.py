@@ -197,11 +197,11 @@ def _cpu_glm_hmc(x, y, chains, L, eps, transitions, min_ess, budget_s,
 
 
 # ------------------------------------------------ C2 large-batch MFMA HMC
-# HBM bytes per all-chain gradient of glm_grad_mfma<4> at 65536 x 256 x 4096:
-# rocprofv3 FETCH_SIZE 265 300 KiB x 2.00 + WRITE_SIZE 32 863 KiB x 1.00 per
-# dispatch, the factors being what the counters read for a 256 MiB device
-# copy (profiles/glm_grad_mfma_logistic_65536x256_counters.md)
-C2_HBM_BYTES_PER_GRADIENT = (265300 * 2.0 + 32863 * 1.0) * 1024
+# HBM bytes per all-chain gradient of glm_grad_mfma<4, false> at 65536 x 256 x
+# 4096: rocprofv3 FETCH_SIZE 265 346 KiB x 2.00 + WRITE_SIZE 32 768 KiB x 1.00
+# per dispatch, the factors being what the counters read for a 256 MiB device
+# copy (profiles/glm_grad_mfma_32x32x16_counters.md)
+C2_HBM_BYTES_PER_GRADIENT = (265346 * 2.0 + 32768 * 1.0) * 1024
 def logistic_65536x256(args, torch, pa):
   from probability_amd import workloads
   n, d, c, L = 65536, 256, 4096, 20

@@ -19,8 +19,9 @@
 // As float64 library operations (two transforms of every series, complex
 // products, copies, a cumulative sum: some forty passes over 65 to 270 MB at
 // 1000 x 64 x 127 float32 draws) ESS and split R-hat took 1446 us together;
-// these kernels take 82 (ess_power 36, ess_transpose 20 at 3.2 TB/s,
-// ess_finish 13, the R-hat kernels 17).
+// these kernels take 81 (each alone: ess_power 36, ess_transpose 20 at 3.3
+// TB/s, ess_finish 13, rhat_moments 10, rhat_finish 7; a launch starts under
+// the end of the one before).
 #include <hip/hip_runtime.h>
 
 #include <cmath>

@@ -11,18 +11,18 @@
 //   glm_tile_grad    one block per (tile of chains, range of rows): partial
 //                    gradients and log-likelihoods (or residual sums of
 //                    squares) to a workspace
-//   glm_tile_finish  one wave (or block) per chain: adds the ranges in order, prior and
-//                    bijector terms (log density and gradient out)
+//   glm_tile_finish  one wave (or block) per chain: adds the ranges in order,
+//                    prior and bijector terms (log density and gradient out)
 //   glm_tile_step    one wave (or block) per chain: the same sums, then the
 //                    leapfrog / Metropolis-Hastings arithmetic of hmc_kernel
 // Log density and gradient, us, one chain per wave -> tiled (float32): 2048 x
-// 64, 1024 chains 43 -> 18; 6001 x 101, 512 chains 161 -> 29; 8192 x 128, 32
-// chains 212 -> 17; 8192 x 128, 2048 chains 310 -> 105 (82 TFLOP/s of 150 that
-// a large float32 matrix product reaches); float64 8000 x 127, 1000 chains 686
-// -> 132.  Large launches are bound by the matrix instructions and the
-// sigmoids between them, which overlap little (matrix cores 60% busy at the
-// largest); small ones by the two launches and their blocks' fixed part, some
-// 9 us.
+// 64, 1024 chains 39 -> 18; 6001 x 101, 512 chains 161 -> 29; 8192 x 128, 32
+// chains 211 -> 16; 8192 x 128, 2048 chains 305 -> 106 (81 TFLOP/s of 150 that
+// a large float32 matrix product reaches); float64 8000 x 127, 1000 chains 681
+// -> 140.  Large launches are bound by the matrix instructions and the
+// sigmoids between them, which overlap little (matrix cores busy for half of
+// the largest, a third of 6001 x 101, 512 chains); small ones by the two
+// launches and their blocks' fixed part, some 9 us.
 #pragma once
 
 #include "../../include/hipmc.h"
@@ -197,12 +197,12 @@ __device__ __attribute__((always_inline)) inline void glm_tile_rows(
     // rounding error, and a linear model's residual is a small difference of
     // them.  Relative error of its gradient, float32 at 8192 x 128 against
     // float64: one chain 2.8e-6, four parts 1.5e-6, eight 1.2e-6 (the per-chain
-    // pass 1.2e-6); sixteen parts spill (8192 x 128, 2048 chains 95 -> 126 us).
+    // pass 1.2e-6); sixteen parts spill (8192 x 128, 2048 chains a third slower).
     // Float64 at 1024 to 1300 rows near the mode, one chain / four / eight
     // parts, rms error against extended precision over the per-chain pass's:
     // 127 columns 1.98 / 1.07 / 0.87, 96 columns 1.50 / 0.89 / 0.75, 64 columns
     // 1.55 / 0.92 / 0.78; so eight from 97 columns on.  (8000 x 127, 1000
-    // chains 130 / 131 / 141 us, where eight spill; 4000 x 64, 1000 chains 50 /
+    // chains 130 / 131 / 140 us, where eight spill; 4000 x 64, 1000 chains 50 /
     // 49 / 65.)
     constexpr int kSets = S < (sizeof(T) == 4 ? 2 : 7) ? 1 : 2;
     Q lg[NG];
@@ -247,8 +247,8 @@ __device__ __attribute__((always_inline)) inline void glm_tile_rows(
           res[j][i] = r;
         }
     } else if (want_sum || sizeof(T) == 8) {
-      // (float64: the branch below spills, and costs 47 us of 132 a gradient
-      // at 8000 x 127, 1000 chains, more than the log-likelihood it saves)
+      // (float64: the branch below spills, and adds a third to a gradient at
+      // 8000 x 127, 1000 chains, more than the log-likelihood it saves)
 #pragma unroll
       for (int i = 0; i < 4; ++i)
 #pragma unroll

@@ -146,8 +146,8 @@ size_t round256(size_t n) { return (n + 255) & ~(size_t)255; }
 //   at least eight passes of its waves, else 256, none shorter than one pass:
 //   a block's fixed part (coefficients in, partial sums out) costs about two
 //   passes.  Log density and gradient, us, 512 against 256 blocks: 2048 x 64,
-//   1024 chains 19.9 / 17.3; 6001 x 101, 512 chains 30.2 / 28.2; 8192 x 128,
-//   2048 chains 98.7 / 101.6; float64 8000 x 127, 1000 chains 131 / 146.
+//   1024 chains 19.9 / 17.9; 6001 x 101, 512 chains 31.5 / 29.2; 8192 x 128,
+//   2048 chains 106.0 / 109.9; float64 8000 x 127, 1000 chains 140 / 168.
 // They depend on the problem's own sizes and chain count only.
 int plan_tiles(int32_t dtype, int32_t n_obs, int32_t dim_x, int32_t n_chains,
                int32_t dim_stride, bool trajectory, hipmc_glm_plan* p) {

@@ -698,7 +698,7 @@ constexpr bool nuts_queue_apart() {
 // products by one where there is nothing to mask (kBijSlot0SoftplusFull): 236
 // -> 195 vector instructions for 258 elements.  20 transitions of 256 groups,
 // 1024 chains (longest 1023 leaves) 8.15 -> 7.03 ms; 24 ragged regressions x 32
-// chains, 3 draws 4.34 -> 3.79 ms.
+// chains, 3 draws 4.34 -> 3.79 ms on one card (4.5 on another).
 // GLM chains are bound by loads in flight, so their kernel is built for two
 // waves per SIMD (the register budget that allows) and blocks of up to
 // eight waves (one chain shared by a whole CU); the other families keep one
