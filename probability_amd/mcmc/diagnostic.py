@@ -159,7 +159,7 @@ def _ess_one(states, cross_chain_dims, filter_threshold):
   if (cross_chain_dims is not None and number and _on_device(states) and
       states.dim() > 1):
     x = _flatten_chain_dims(states, cross_chain_dims)
-    if x.numel() > 0 and _ess_takes(*_series(x, 1).shape):
+    if x.numel() > 0 and _ess_takes(*x.shape[:2], math.prod(x.shape[2:])):
       return _ess_device(x, filter_threshold)
   states = _as64(states)
   if cross_chain_dims is not None:
